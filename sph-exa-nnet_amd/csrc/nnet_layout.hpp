@@ -8,6 +8,9 @@ namespace nnet_amd
 {
 constexpr int MAXQ  = 3;  // reactant entries per reaction
 constexpr int MAXSP = 88; // species + 1 of the largest network
+// row stride (doubles) of the eight-pivot LU's panel columns: even, so that a row's eight entries
+// are 16-byte aligned, and 20 words over 64 LDS banks spread the 16 rows of a tile evenly
+constexpr int PANEL8 = 10;
 
 // The exp / pow values of the six hand-fitted rate groups, evaluated one per lane of a wavefront:
 // level 1, NE1 exps and NP1 pows; level 2, NE2 exps of level-1 results.  They pass through the
@@ -66,13 +69,18 @@ struct Lds
     static constexpr int oBE = (headEnd > f32Words ? headEnd : f32Words), oDYdot = oBE + D, oDYdT = oDYdot + D,
                          oCorr = oDYdT + D, oEv = oCorr + D, oEos = oEv + 12, oJv = oEos + 4,
                          phaseEnd = oJv + C::NNZ;
-    // the FP64 packed rows alias everything above once the matrix sits in registers
-    static constexpr int unionSize = phaseEnd > NU ? phaseEnd : NU;
+    // the FP64 packed rows alias everything above once the matrix sits in registers; the
+    // eight-pivot LU (net86 / net87, FP64) stores them with the tiles' padding columns
+    static constexpr int NPAD = 16 * C::TT;
+    static constexpr bool LU8 = C::TT > 1 && !MIX;
+    static constexpr int uWords = LU8 ? NPAD * (NPAD - 1) / 2 : NU;
+    static constexpr int unionSize = phaseEnd > uWords ? phaseEnd : uWords;
     static constexpr int oY = unionSize, oYb = oY + D, oX = oYb + D, oRow0 = oX + N + 1;
     // LU panel buffers (two generations of: panel columns [row][4], pivot rows [column][4]); after
-    // the LU they hold the refinement residual
-    static constexpr int NPAD = 16 * C::TT, oPan = ((oRow0 + (MIX ? N + 1 : 0)) + 3) & ~3,
-                         total = oPan + 16 * NPAD;
+    // the LU they hold the refinement residual.  Eight-pivot LU: two generations of panel columns
+    // [row][PANEL8] (its pivot rows go straight into the packed rows).
+    static constexpr int oPan = ((oRow0 + (MIX ? N + 1 : 0)) + 3) & ~3, panWords = (LU8 ? 2 * PANEL8 : 16) * NPAD,
+                         total = oPan + panWords;
 };
 
 // Jacobian non-zero slot (position in the image's descending-length order) that lane `tid` of a
@@ -120,5 +128,25 @@ struct LuIdx
     // A-operand row m of a tile: FP64 MFMA rows come in result order; the FP32 MFMA returns row
     // 4(l>>4) + v in register v, so with the FP64 placement A-operand row m is (m>>2) + 4(m&3)
     static constexpr int arow(bool fp32, int m) { return fp32 ? (m >> 2) + 4 * (m & 3) : m; }
+};
+
+// Index functions of the eight-pivot LU (net86 / net87, FP64): block B eliminates pivots 8B ..
+// 8B + 7 (B even: the first half of tile row / column B/2, B odd: the second half).
+template<int NET>
+struct Lu8Idx
+{
+    using C = Cfg<NET>;
+    static constexpr int N = C::N, NPAD = 16 * C::TT;
+    static constexpr int NB = (N + 7) / 8; // blocks
+    // panel column q of block B in generation (B & 1) of the panel buffers
+    static constexpr int pcol(int B, int row, int q) { return (B & 1) * PANEL8 * NPAD + row * PANEL8 + q; }
+    // normalised upper entry (k, j), k < j < NPAD, packed by columns as LuIdx::uidx packs it
+    static constexpr int uidx(int k, int j) { return j * (j - 1) / 2 + k; }
+    // waves that hold trailing rows (lane row 8B + 8 + 64 w + lane) and columns (lane column 8B +
+    // 1 + 64 w + lane, so that the block's own columns are normalised by the same lanes)
+    static constexpr int row0(int B) { return 8 * B + 8; }
+    static constexpr int col0(int B) { return 8 * B + 1; }
+    static constexpr int rowWaves(int B) { return row0(B) >= N ? 0 : (N - row0(B) + 63) / 64; }
+    static constexpr int colWaves(int B) { return (N + 1 - col0(B) + 63) / 64; }
 };
 } // namespace nnet_amd

@@ -29,6 +29,7 @@
 #include <mutex>
 #include <string>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "../../include/nnet_mi355x.h"
@@ -587,6 +588,248 @@ struct TileLU
                 }
             }
         }
+    }
+};
+
+// value of x in lane K of each 16-lane row of the wavefront
+template<int K>
+__device__ __forceinline__ double row_bcast(double x)
+{
+    return __builtin_amdgcn_update_dpp(0., x, 0x150 + K, 0xf, 0xf, true); // row_newbcast:K
+}
+template<int... I, class F>
+__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template<int N, class F>
+__device__ __forceinline__ void static_for(F&& f)
+{
+    static_for_impl(std::make_integer_sequence<int, N>{}, f);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Eight-pivot LU of the FP64 net86 / net87 solve, on the same register tiles as TileLU and with
+// the same arithmetic per element (pivots in ascending order, one fma each; multipliers with
+// |w| <= 1e-40 count as zero), so its factors are those of the four-pivot blocks.
+//
+// The factorization's time is not its operations but the chain of its blocks: LDS round trips, two
+// barriers and the diagonal block's dependent steps, at one wavefront per SIMD and particle.
+// Blocks of eight halve the number of round trips and barriers (11 blocks instead of 22), and the
+// diagonal block costs few instructions: it is held one row per lane of a 16-lane row (replicated
+// over the wavefront) and the pivot row reaches the others through DPP row broadcasts, instead
+// of a 4x4 block unrolled into every lane's registers.  Wavefronts 0-1 hold the trailing rows and
+// 2-3 the trailing columns, one per lane; the normalised rows are stored where the back
+// substitution reads them, so the panel buffers hold panel columns only.
+// ---------------------------------------------------------------------------------------------
+template<int NET>
+struct PanelLU
+{
+    using C = Cfg<NET>;
+    using X = Lu8Idx<NET>;
+    static constexpr int N = C::N, TT = C::TT, WR = C::WR, TI = TT / WR;
+    static_assert(WR == 2 && C::NT == 256 && 16 * TT > N && TT % WR == 0, "2 x 2 wavefronts");
+
+    // the owners of block B's columns and rows store them: panel columns (rows of tile rows >= Tp)
+    // to the panel buffer, the pivot rows right of the diagonal to the packed rows
+    template<int B>
+    static __device__ __forceinline__ void publish(const dx4 (&Mt)[TI][TI], double* pan, double* sU, int wr, int wc,
+                                                   int lr, int lc)
+    {
+        constexpr int p0 = 8 * B, Tp = p0 >> 4, c0 = p0 & 15, v0 = c0 >> 2;
+        // (rows above the panel are stored too: nothing reads them, and the test would cost a branch)
+        if (wc == Tp % WR && (lc >> 3) == (c0 >> 3))
+        {
+            double* o = pan + X::pcol(B, 16 * wr + lr, lc - c0);
+#pragma unroll
+            for (int ti = Tp / WR; ti < TI; ++ti)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    o[(16 * WR * ti + 4 * v) * PANEL8] = Mt[ti][Tp / WR][v];
+        }
+        if (wr == Tp % WR)
+        {
+#pragma unroll
+            for (int tj = Tp / WR; tj < TI; ++tj)
+            {
+                const int col = tile_col(wc + WR * tj, lc);
+                double*   o   = sU + X::uidx(p0 + lr, col);
+                // only the first tile column holds columns left of the diagonal
+                if (tj > Tp / WR || col > p0 + lr) o[0] = Mt[Tp / WR][tj][v0];
+                if (tj > Tp / WR || col > p0 + lr + 4) o[4] = Mt[Tp / WR][tj][v0 + 1];
+            }
+        }
+    }
+
+    // pivot q of the diagonal block: its normalised row entry right of the diagonal, broadcast from
+    // lane q, to upd(c, u) column by column; rinv: the pivot's reciprocal on entry, the next
+    // pivot's on exit.  The next pivot's column comes first and its reciprocal (the dependent
+    // chain of the block) is started before the other columns.
+    template<int q, class F>
+    static __device__ __forceinline__ void normalised(const double (&a)[8], double& rinv, F&& upd)
+    {
+        if constexpr (q < 7)
+        {
+            double t[8];
+#pragma unroll
+            for (int c = q + 1; c < 8; ++c)
+                t[c] = a[c] * rinv;
+            upd(q + 1, row_bcast<q>(t[q + 1]));
+            const double d = row_bcast<q + 1>(a[q + 1]);
+            double       u[8];
+#pragma unroll
+            for (int c = q + 2; c < 8; ++c)
+                u[c] = row_bcast<q>(t[c]);
+            rinv = TileT<double>::recip(d);
+#pragma unroll
+            for (int c = q + 2; c < 8; ++c)
+                upd(c, u[c]);
+        }
+    }
+
+    template<int B>
+    static __device__ __forceinline__ void step(dx4 (&Mt)[TI][TI], double* pan, double* sU, int w, int lane)
+    {
+        constexpr int    p0 = 8 * B, Tp = p0 >> 4, c0 = p0 & 15, nq = N - p0 < 8 ? N - p0 : 8;
+        constexpr double eps = k::epsilonSystem;
+        // an opaque lane index (range restored): the block's addresses are formed here, not kept
+        // live from the kernel entry for all blocks
+        asm volatile("" : "+v"(lane));
+        lane &= 63;
+        const int  wr = w / WR, wc = w % WR, lr = lane >> 4, lc = lane & 15;
+        const bool rows = w < X::rowWaves(B), cols = w >= 2 && w - 2 < X::colWaves(B);
+
+        if (rows || cols)
+        {
+            // diagonal block: row p0 + (lane & 7) in this lane
+            double        a[8];
+            const double* d = pan + X::pcol(B, p0 + (lane & 7), 0);
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+                a[c] = d[c];
+            if (rows)
+            {
+                // one lane per trailing row: its eight multipliers, negated (the update's A operand),
+                // in place of its panel entries
+                const int i = X::row0(B) + 64 * w + lane;
+                double*   P = pan + X::pcol(B, i < N ? i : N - 1, 0);
+                double    pr[8];
+#pragma unroll
+                for (int c = 0; c < 8; ++c)
+                    pr[c] = P[c];
+                double rinv = TileT<double>::recip(row_bcast<0>(a[0]));
+                static_for<8>(
+                    [&](auto qc) __attribute__((always_inline))
+                    {
+                        constexpr int q  = decltype(qc)::value;
+                        const double  wd = fabs(a[q]) > eps ? -a[q] : -0.;
+                        const double  wp = fabs(pr[q]) > eps ? -pr[q] : -0.;
+                        pr[q]            = wp;
+                        normalised<q>(a, rinv,
+                                      [&](int c, double u) __attribute__((always_inline))
+                                      {
+                                          a[c]  = fma(wd, u, a[c]);
+                                          pr[c] = fma(wp, u, pr[c]);
+                                      });
+                    });
+                if (i < N)
+#pragma unroll
+                    for (int c = 0; c < 8; ++c)
+                        P[c] = pr[c];
+            }
+            else
+            {
+                // one lane per column right of the diagonal: the normalised pivot-row entries, in
+                // place (a column of the block itself takes those above its diagonal)
+                const int j = X::col0(B) + 64 * (w - 2) + lane;
+                double*   U = sU + X::uidx(p0, j <= N ? j : N);
+                double    cu[8];
+#pragma unroll
+                for (int q = 0; q < nq; ++q)
+                    cu[q] = U[q];
+                double rinv = TileT<double>::recip(row_bcast<0>(a[0]));
+                static_for<nq>(
+                    [&](auto qc) __attribute__((always_inline))
+                    {
+                        constexpr int q  = decltype(qc)::value;
+                        const double  wd = fabs(a[q]) > eps ? -a[q] : -0.;
+                        cu[q] *= rinv;
+                        normalised<q>(a, rinv,
+                                      [&](int c, double u) __attribute__((always_inline)) { a[c] = fma(wd, u, a[c]); });
+                        static_for<nq - (q + 1)>(
+                            [&](auto cc) __attribute__((always_inline))
+                            {
+                                constexpr int r = q + 1 + decltype(cc)::value;
+                                cu[r]           = fma(row_bcast<r>(wd), cu[q], cu[r]);
+                            });
+                    });
+                if (j <= N)
+#pragma unroll
+                    for (int q = 0; q < nq; ++q)
+                        if (p0 + q < j) U[q] = cu[q];
+            }
+        }
+        __syncthreads();
+        if constexpr (X::rowWaves(B) > 0)
+        {
+            // rank-8 trailing update, two MFMAs per tile (A operand: row l&15 of the tile, pivot
+            // 4s + (l>>4); B operand: pivot 4s + (l>>4), column l&15).  Rows and columns that are
+            // already eliminated, and the padding, take part with whatever their operands hold:
+            // nothing reads their registers again.  The tiles of the next block's panel first
+            // (as in TileLU), then its publish, then the others.
+            constexpr int T0 = Tp + (c0 ? 1 : 0), t0 = T0 / WR; // the next panel's tile row / column
+            double        Aop[TI][2], Bop[TI][2];
+            const double* pa = pan + X::pcol(B, 16 * wr + lc, lr);
+#pragma unroll
+            for (int ti = t0; ti < TI; ++ti)
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+                    Aop[ti][s] = pa[16 * WR * ti * PANEL8 + 4 * s];
+#pragma unroll
+            for (int tj = t0; tj < TI; ++tj)
+            {
+                const double* pb = sU + X::uidx(p0 + lr, tile_col(wc + WR * tj, lc));
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+                    Bop[tj][s] = pb[4 * s];
+            }
+            auto tile = [&](int ti, int tj) __attribute__((always_inline))
+            {
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+                    Mt[ti][tj] = TileT<double>::mfma(Aop[ti][s], Bop[tj][s], Mt[ti][tj]);
+            };
+            // a wavefront's tiles t0 lie in the panel or, with T0 odd, may be eliminated already
+            const bool r0 = wr + WR * t0 >= T0, q0 = wc + WR * t0 >= T0;
+            if (r0 && q0) tile(t0, t0);
+            if (r0)
+#pragma unroll
+                for (int tj = t0 + 1; tj < TI; ++tj)
+                    tile(t0, tj);
+            if (q0)
+#pragma unroll
+                for (int ti = t0 + 1; ti < TI; ++ti)
+                    tile(ti, t0);
+            publish<B + 1>(Mt, pan, sU, wr, wc, lr, lc);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int ti = t0 + 1; ti < TI; ++ti)
+#pragma unroll
+                for (int tj = t0 + 1; tj < TI; ++tj)
+                    tile(ti, tj);
+            __syncthreads();
+        }
+        if constexpr (B + 1 < X::NB) step<B + 1>(Mt, pan, sU, w, lane);
+    }
+
+    // forward elimination of the augmented matrix; leaves the normalised rows in sU (the caller has
+    // every lane's matrix in its registers: sU overwrites the arrays it was built from)
+    static __device__ __forceinline__ void factor(dx4 (&Mt)[TI][TI], double* pan, double* sU, int w, int lane)
+    {
+        __syncthreads();
+        publish<0>(Mt, pan, sU, w / WR, w % WR, lane >> 4, lane & 15);
+        __syncthreads();
+        step<0>(Mt, pan, sU, w, lane);
     }
 };
 
@@ -1301,7 +1544,10 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
                 // the LU's first panel publish (which writes only the panel buffers) orders every
                 // lane's fill before the first packed-row store
                 // ---- LU (eigen.hpp:179-206), four pivots per block ----
-                TileLU<NET, double, false, WAVE>::factor(Mt, sPan, sU, nullptr, nullptr, wr, wc, lr, lc, tid);
+                if constexpr (L::LU8)
+                    PanelLU<NET>::factor(Mt, sPan, sU, __builtin_amdgcn_readfirstlane(tid >> 6), tid & 63);
+                else
+                    TileLU<NET, double, false, WAVE>::factor(Mt, sPan, sU, nullptr, nullptr, wr, wc, lr, lc, tid);
                 // ---- back substitution (eigen.hpp:208-221) ----
                 if (tid < 64)
                 {
