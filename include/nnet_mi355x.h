@@ -166,9 +166,11 @@ int nnet_compute_noalloc(nnet_ctx* ctx, const nnet_batch* batches, int nb, doubl
                          double previous_dt, int use_drhodt, void* stream);
 
 /* Cap on Newton iterations per particle per call (default 10000; 0 = no cap).  The reference
- * controller can also cycle between two rejected timesteps for thousands of attempts before (or
+ * controller can also cycle between rejected timesteps for thousands of attempts before (or
  * instead of) accepting one; the cap bounds that work.  A capped particle is left at its last
- * accepted substep with status NNET_STATUS_MAX_ITER. */
+ * accepted substep with status NNET_STATUS_MAX_ITER.  Attempts that repeat bit for bit are run for
+ * one period and counted for the rest, so the state, the timestep and the counts are those of
+ * running every iteration up to the cap. */
 int nnet_ctx_set_max_iterations(nnet_ctx* ctx, long max_iter);
 
 /* Particles a solve launch integrates concurrently on this context's device: the workgroups of

@@ -3,6 +3,7 @@
 // same definitions compile into the device code and into host-side checks of every LDS index
 // the kernels form (clang treats constexpr functions as host and device functions).
 #pragma once
+#include <cstdint>
 
 namespace nnet_amd
 {
@@ -80,8 +81,46 @@ struct Lds
     // the LU they hold the refinement residual.  Eight-pivot LU: two generations of panel columns
     // [row][PANEL8] (its pivot rows go straight into the packed rows).
     static constexpr int oPan = ((oRow0 + (MIX ? N + 1 : 0)) + 3) & ~3, panWords = (LU8 ? 2 * PANEL8 : 16) * NPAD,
-                         total = oPan + panWords;
+                         oCyc = oPan + panWords, total = oCyc + 3 * (C::NT / 64); // a Cycle per wavefront
 };
+
+// Exact cycles of rejected attempts.  A rejected attempt restarts from the same accepted state, so
+// all that follows until the next acceptance is a function of the attempt's (dt, T_buffer) alone:
+// when a pair comes back bit for bit, the attempts between the two visits repeat until the
+// Newton-iteration cap.  A pair that comes back at once is status STALLED; for longer periods the
+// controller counts the whole periods that fit under the cap and runs only the rest, ending in the
+// state and with the counts that running them all ends in.  The pair kept for comparison is
+// replaced after windows of doubled length (Brent, BIT 20, 176, 1980), which finds any period
+// within a few times max(period, lead-in).
+struct Cycle
+{
+    uint64_t dt, Tb;  // bits of the kept pair
+    uint32_t it, lim; // iteration at which it was kept, length of its window (0: none kept)
+};
+static_assert(sizeof(Cycle) == 24, "three LDS doubles");
+
+// After a rejection at iteration `total` that leaves the pair (dt, Tb): the iterations of whole
+// periods to count without running them (0: no period known).  At least one iteration is left
+// to run, so the cap ends the particle as it always does.
+__attribute__((always_inline)) constexpr long cycle_skip(Cycle& c, uint64_t dt, uint64_t Tb, long total, long max_iter)
+{
+    const uint32_t since = (uint32_t)total - c.it;
+    if (c.lim != 0 && c.dt == dt && c.Tb == Tb)
+    {
+        const long     rem  = max_iter - 1 - total; // max_iter <= 0: no cap
+        const uint32_t skip = rem > 0 ? (uint32_t)(rem < 0x7fffffffL ? rem : 0x7fffffffL) / since * since : 0;
+        c.it += skip;
+        return (long)skip;
+    }
+    if (c.lim == 0 || since >= c.lim)
+    {
+        c.dt  = dt;
+        c.Tb  = Tb;
+        c.it  = (uint32_t)total;
+        c.lim = c.lim == 0 ? 1 : c.lim < 0x40000000u ? 2 * c.lim : c.lim;
+    }
+    return 0;
+}
 
 // Jacobian non-zero slot (position in the image's descending-length order) that lane `tid` of a
 // particle's NT lanes sums in pass `pass`, or a value >= nnz when it has none: pass p takes slot

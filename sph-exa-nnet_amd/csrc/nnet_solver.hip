@@ -891,6 +891,8 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
     double* sX    = sm + L::oX;
     double* sPan  = sm + L::oPan;
     double* sRow0 = sm + L::oRow0;
+    // this wavefront's own copy (each wavefront runs the controller, none waits for another there)
+    Cycle& cyc = reinterpret_cast<Cycle*>(sm + L::oCyc)[tid >> 6];
 
     const int lr = (tid & 63) >> 4, lc = tid & 15, wr = (tid >> 6) / WR, wc = (tid >> 6) % WR;
 
@@ -955,6 +957,7 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
         uint32_t     n_sub = 0, n_newton = 0;
         bool         abandon = false; // mixed pass: FP32 refinement failed, left to the FP64 redo pass
         uint8_t      status = NNET_STATUS_OK;
+        cyc.lim             = 0;
 
         for (int i = 1;; ++i)
         {
@@ -1738,6 +1741,7 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
                 i = 0;
                 elapsed += timestep;
                 ++n_sub;
+                cyc.lim = 0;
                 if ((dt_tot - elapsed) / dt_tot < k::substep_dtTol) break;
             }
             else if (i == 0)
@@ -1749,6 +1753,14 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
                     status = NNET_STATUS_STALLED;
                     break;
                 }
+                // longer exact cycles: their whole periods are counted, not run.  Most particles
+                // that reach the cap are in one: of the Newton iterations of net14, net86 and net87
+                // Helmholtz samples at cap 10,000, whole periods hold 62%, 62% and 82%.  524,288
+                // net86 particles, first step: 787 -> 592 ms; 50,021 net14 particles: 738 -> 527 ms.
+                const long skip = cycle_skip(cyc, (uint64_t)__double_as_longlong(dt),
+                                             (uint64_t)__double_as_longlong(T_buf), total_iter, sp.max_iter);
+                total_iter += skip;
+                n_newton += (uint32_t)skip;
             }
             if (sp.max_iter > 0 && total_iter >= sp.max_iter)
             {
