@@ -66,12 +66,14 @@ struct Lds
                          oTr = oDval + NR, oJok = oTr + NR * MAXQ, headEnd = oJok + NR;
     // FP32 factors of the mixed path (U rows, multipliers, pivot reciprocals), in doubles
     static constexpr int f32Words = MIX ? (NU + NL + N + 1) / 2 : 0;
-    // tail: what the matrix fill and the FP64 refinement residual read
-    static constexpr int oBE = (headEnd > f32Words ? headEnd : f32Words), oDYdot = oBE + D, oDYdT = oDYdot + D,
+    // tail: what the matrix fill and the FP64 refinement residual read; behind the factors, because
+    // the next iteration reads it again when it linearises at the same state
+    static constexpr int factorEnd = MIX ? f32Words : NU;
+    static constexpr int oBE = (headEnd > factorEnd ? headEnd : factorEnd), oDYdot = oBE + D, oDYdT = oDYdot + D,
                          oCorr = oDYdT + D, oEv = oCorr + D, oEos = oEv + 12, oJv = oEos + 4,
                          phaseEnd = oJv + C::NNZ;
-    // the FP64 packed rows alias everything above once the matrix sits in registers; the
-    // eight-pivot LU (net86 / net87, FP64) stores them with the tiles' padding columns
+    // the FP64 packed rows alias the head once the matrix sits in registers; the eight-pivot LU's
+    // (net86 / net87, FP64) operand loads also address the tiles' padding columns behind them
     static constexpr int NPAD = 16 * C::TT;
     static constexpr bool LU8 = C::TT > 1 && !MIX;
     static constexpr int uWords = LU8 ? NPAD * (NPAD - 1) / 2 : NU;

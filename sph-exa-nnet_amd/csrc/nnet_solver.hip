@@ -654,9 +654,11 @@ struct PanelLU
             {
                 const int col = tile_col(wc + WR * tj, lc);
                 double*   o   = sU + X::uidx(p0 + lr, col);
-                // only the first tile column holds columns left of the diagonal
-                if (tj > Tp / WR || col > p0 + lr) o[0] = Mt[Tp / WR][tj][v0];
-                if (tj > Tp / WR || col > p0 + lr + 4) o[4] = Mt[Tp / WR][tj][v0 + 1];
+                // only the first tile column holds columns left of the diagonal; only the last tile
+                // holds padding columns (not stored: the arrays behind the packed rows stay)
+                const bool in = 16 * (WR * tj + WR) <= N + 1 || col <= N;
+                if (in && (tj > Tp / WR || col > p0 + lr)) o[0] = Mt[Tp / WR][tj][v0];
+                if (in && (tj > Tp / WR || col > p0 + lr + 4)) o[4] = Mt[Tp / WR][tj][v0 + 1];
             }
         }
     }
@@ -958,6 +960,7 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
         bool         abandon = false; // mixed pass: FP32 refinement failed, left to the FP64 redo pass
         uint8_t      status = NNET_STATUS_OK;
         cyc.lim             = 0;
+        bool         kept = false; // the assembly arrays are those of the accepted state
 
         for (int i = 1;; ++i)
         {
@@ -978,467 +981,478 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
             // prepareSystemNR (nuclear_net.hpp:699-712)
             const double T_loc   = (i <= 1) ? T : T_buf;
             const double T_theta = (1 - k::theta) * T + k::theta * T_loc;
-            for (int s = tid; s < D; s += NT)
+            // A rejected attempt restarts from the accepted state, and its first iteration linearises
+            // there whatever its timestep: rates, EOS, Jacobian and their sums are those of the attempt
+            // before it, still in the assembly arrays when that one was rejected in its first iteration
+            // too (a later iteration or another state has written them otherwise).  Such an iteration
+            // is the matrix fill and the solve alone, and most iterations of a capped particle are of
+            // this kind.  50,021 net14 particles, first step: 533 -> 84 ms; 4,099 of net87, whose
+            // attempts mostly fail later: unchanged (93 ms).
+            const bool  again = kept && i == 1;
+            const uint4 lmap  = nd.lanemap[tid]; // register-slot mask, first non-zero id (matrix fill)
+            kept              = i == 1;
+            if (!again)
             {
-                const double yb = (i <= 1) ? sY[s] : sYb[s];
-                sYb[s]          = (1 - k::theta) * sY[s] + k::theta * yb;
-            }
-            psync<WAVE>();
-
-            // ---- EOS (one lane) and rates, phase 1 (all lanes) ----
-            if constexpr (EOSK != NNET_EOS_IDEAL)
-            {
-                if (tid == NT - 1)
+                for (int s = tid; s < D; s += NT)
                 {
-                    // helmholtz.hpp:221-222: sum(Y) and sum(Y Z), each in index order; eight
-                    // abundances are loaded ahead of the two interleaved addition chains
-                    double abar = 0., zbar = 0;
-                    int    s    = 0;
-                    for (; s + 8 <= ed.zdim; s += 8)
+                    const double yb = (i <= 1) ? sY[s] : sYb[s];
+                    sYb[s]          = (1 - k::theta) * sY[s] + k::theta * yb;
+                }
+                psync<WAVE>();
+
+                // ---- EOS (one lane) and rates, phase 1 (all lanes) ----
+                if constexpr (EOSK != NNET_EOS_IDEAL)
+                {
+                    if (tid == NT - 1)
                     {
-                        double y[8];
-#pragma unroll
-                        for (int u = 0; u < 8; ++u)
-                            y[u] = sYb[s + u];
-                        __builtin_amdgcn_sched_barrier(0); // keep the eight loads in flight together
-#pragma unroll
-                        for (int u = 0; u < 8; ++u)
+                        // helmholtz.hpp:221-222: sum(Y) and sum(Y Z), each in index order; eight
+                        // abundances are loaded ahead of the two interleaved addition chains
+                        double abar = 0., zbar = 0;
+                        int    s    = 0;
+                        for (; s + 8 <= ed.zdim; s += 8)
                         {
-                            abar += y[u];
-                            zbar += y[u] * ed.Z[s + u];
+                            double y[8];
+#pragma unroll
+                            for (int u = 0; u < 8; ++u)
+                                y[u] = sYb[s + u];
+                            __builtin_amdgcn_sched_barrier(0); // keep the eight loads in flight together
+#pragma unroll
+                            for (int u = 0; u < 8; ++u)
+                            {
+                                abar += y[u];
+                                zbar += y[u] * ed.Z[s + u];
+                            }
+                        }
+                        for (; s < ed.zdim; ++s)
+                        {
+                            abar += sYb[s];
+                            zbar += sYb[s] * ed.Z[s];
+                        }
+                        double c0, d0;
+                        helmholtz_cv_dpdt(ed.grid, ed.cells, abar, zbar, T_theta, rho_t, c0, d0);
+                        sEos[0] = c0;
+                        sEos[1] = d0;
+                    }
+                }
+                {
+                    const double Tg = T_theta;
+                    const int    SS = nd.nfit; // species lanes follow the fitted-rate lanes
+                    if (tid < nd.nfit)
+                    {
+                        const int     f  = tid;
+                        const double* fc = nd.fit + 8 * f;
+                        const double  t9 = Tg / 1.e9, t913 = pow(t9, 1. / 3.), t923 = t913 * t913, t953 = pow(t9, 5. / 3.);
+                        const double  t9i = 1.e0 / t9, t9i2 = t9i * t9i, t9i13 = 1.e0 / t913, t9i23 = t9i13 * t9i13,
+                                     t9i43 = t9i23 * t9i23, lt9 = log(t9);
+                        const double coef =
+                            fc[1] * t9i + fc[2] * t9i13 + fc[3] * t913 + fc[4] * t9 + fc[5] * t953 + fc[6] * lt9;
+                        const double dcoef =
+                            (-fc[1] * t9i2 + (-fc[2] * t9i43 + fc[3] * t9i23 + 5 * fc[5] * t923) * (1. / 3.) + fc[4] +
+                             fc[6] * t9i) *
+                            1e-9;
+                        const int    e   = nd.fit_e0 + f;
+                        const double eff = exp(fc[0] + coef);
+                        sEff[e]          = eff;
+                        sDeff[e]         = eff * dcoef;
+                        // reverse rate (net14.cpp:150-190, net86.cpp:524-554)
+                        const double rt9  = nd.rev_div ? Tg / 1.e9 : Tg * 1e-09;
+                        const double rt9i = 1. / rt9;
+                        const double val1 = 11.6045 * rt9i;
+                        const double val3 = val1 * rt9i * 1e-9;
+                        const int    kb   = temperature_bin(Tg);
+                        const double part = nd.choose[nd.ca[f] * 24 + kb] / nd.choose[nd.cb[f] * 24 + kb];
+                        double       l, dl;
+                        if (nd.photo[f])
+                        {
+                            const double val2 = 1.5 * log(rt9);
+                            const double val4 = 1.5e-9 * rt9i;
+                            l                 = part * exp(fc[7] + coef - val1 * nd.q[f] + val2);
+                            dl                = l * (dcoef + val3 * nd.q[f] + val4);
+                        }
+                        else
+                        {
+                            l  = part * exp(fc[7] + coef - val1 * nd.q[f]);
+                            dl = l * (dcoef + val3 * nd.q[f]);
+                        }
+                        sL[e]  = l;
+                        sDl[e] = dl;
+                    }
+                    else if (tid >= SS && tid < SS + Dr)
+                    {
+                        // corrected binding energy (net14.cpp:49-75) and screening mu/kT (:577-600)
+                        const int    s          = tid - SS;
+                        const double kbt        = phys::Kb * Tg;
+                        const double nakbt      = phys::Na * kbt;
+                        const double correction = -1.5 * nakbt;
+                        const double ne         = rho_t * phys::Na / 2.;
+                        {
+                            const double ae  = pow((3. / 4.) / (phys::pi * ne), 1. / 3.);
+                            const double gam = phys::e2 / (kbt * ae);
+                            const double gmm = gam * nd.Z53[s];
+                            const double fn  = gmm > 1 ? coulomb_strong(gmm) : coulomb_weak(gmm);
+                            double       be  = nd.BE0[s] + correction;
+                            be -= nakbt * fn;
+                            sBE[s] = be;
+                        }
+                        {
+                            const double kbt2 = Tg * phys::Kb;
+                            const double ae   = pow(3. / (4. * phys::pi * ne), 1. / 3.);
+                            const double gam  = phys::e2 / (kbt2 * ae);
+                            const double a1 = -.898004, b1 = .96786, c1 = .220703, d1 = -.86097, e1 = 2.520058332;
+                            const double gp  = gam * nd.Z53[s];
+                            const double sq  = sqrt(gp);
+                            const double sq2 = sqrt(sq);
+                            double       mu;
+                            if (gp <= 1)
+                                mu = -(1. / 1.7320508075688772) * gp * sq + pow(gp, 1.9885) * .29561 / 1.9885;
+                            else
+                                mu = a1 * gp + 4. * (b1 * sq2 - c1 / sq2) + d1 * log(gp) - e1;
+                            if (NET != 14 && s == 1) mu = 0; // neutron (net86.cpp:603)
+                            sMu[s] = mu;
                         }
                     }
-                    for (; s < ed.zdim; ++s)
+                    // hand-fitted rates.  net14: the groups' exp / pow values spread over the lanes of
+                    // its one wavefront, then combined in every lane; net86 / net87: one group per lane
+                    // on lanes of different wavefronts (measured faster there than the lane-parallel
+                    // form on one of their wavefronts)
+                    if constexpr (NET == 14)
                     {
-                        abar += sYb[s];
-                        zbar += sYb[s] * ed.Z[s];
-                    }
-                    double c0, d0;
-                    helmholtz_cv_dpdt(ed.grid, ed.cells, abar, zbar, T_theta, rho_t, c0, d0);
-                    sEos[0] = c0;
-                    sEos[1] = d0;
-                }
-            }
-            {
-                const double Tg = T_theta;
-                const int    SS = nd.nfit; // species lanes follow the fitted-rate lanes
-                if (tid < nd.nfit)
-                {
-                    const int     f  = tid;
-                    const double* fc = nd.fit + 8 * f;
-                    const double  t9 = Tg / 1.e9, t913 = pow(t9, 1. / 3.), t923 = t913 * t913, t953 = pow(t9, 5. / 3.);
-                    const double  t9i = 1.e0 / t9, t9i2 = t9i * t9i, t9i13 = 1.e0 / t913, t9i23 = t9i13 * t9i13,
-                                 t9i43 = t9i23 * t9i23, lt9 = log(t9);
-                    const double coef =
-                        fc[1] * t9i + fc[2] * t9i13 + fc[3] * t913 + fc[4] * t9 + fc[5] * t953 + fc[6] * lt9;
-                    const double dcoef =
-                        (-fc[1] * t9i2 + (-fc[2] * t9i43 + fc[3] * t9i23 + 5 * fc[5] * t923) * (1. / 3.) + fc[4] +
-                         fc[6] * t9i) *
-                        1e-9;
-                    const int    e   = nd.fit_e0 + f;
-                    const double eff = exp(fc[0] + coef);
-                    sEff[e]          = eff;
-                    sDeff[e]         = eff * dcoef;
-                    // reverse rate (net14.cpp:150-190, net86.cpp:524-554)
-                    const double rt9  = nd.rev_div ? Tg / 1.e9 : Tg * 1e-09;
-                    const double rt9i = 1. / rt9;
-                    const double val1 = 11.6045 * rt9i;
-                    const double val3 = val1 * rt9i * 1e-9;
-                    const int    kb   = temperature_bin(Tg);
-                    const double part = nd.choose[nd.ca[f] * 24 + kb] / nd.choose[nd.cb[f] * 24 + kb];
-                    double       l, dl;
-                    if (nd.photo[f])
-                    {
-                        const double val2 = 1.5 * log(rt9);
-                        const double val4 = 1.5e-9 * rt9i;
-                        l                 = part * exp(fc[7] + coef - val1 * nd.q[f] + val2);
-                        dl                = l * (dcoef + val3 * nd.q[f] + val4);
+                        if ((tid >> 6) == 0)
+                        {
+                            // the values pass through the Jacobian array, which is rewritten only after
+                            // this phase: sJv[0 .. N1) level 1, sJv[N1 .. N1 + NE2) level 2
+                            static_assert(C::NNZ >= spx::N1 + spx::NE2, "hand-fitted values fit the Jacobian array");
+                            const int      k = tid & 63;
+                            const RatePow  p(Tg);
+                            const DerivPow q(Tg);
+                            {
+                                const double t1 = special_level1(k, p, q);
+                                if (k < spx::N1) sJv[k] = t1;
+                            }
+                            psync<true>(); // one wavefront
+                            auto v1 = [&](int j) __attribute__((always_inline)) -> double { return sJv[j]; };
+                            {
+                                const double t2 = special_level2(k, p, q, v1);
+                                if (k < spx::NE2) sJv[spx::N1 + k] = t2;
+                            }
+                            psync<true>();
+                            auto v2 = [&](int j) __attribute__((always_inline)) -> double { return sJv[spx::N1 + j]; };
+                            // lane 0 stores each group's rate (and reverse) with its derivative
+                            auto store = [&](int g, double r, double rl, double dr, double drl) __attribute__((always_inline))
+                            {
+                                if (k != 0) return;
+                                const int e = g == 0 ? nd.sp.r3a_e : g == 1 ? nd.sp.r24 : g == 2 ? nd.sp.r1216 : g == 3 ? nd.sp.r32
+                                            : g == 4 ? nd.sp.rcag_e : nd.sp.roag_e;
+                                sEff[e]  = r;
+                                sDeff[e] = dr;
+                                if (g == 0 || g >= 4)
+                                {
+                                    const int l = g == 0 ? nd.sp.r3a_l : g == 4 ? nd.sp.rcag_l : nd.sp.roag_l;
+                                    sL[l]       = rl;
+                                    sDl[l]      = drl;
+                                }
+                            };
+                            special_combine(Tg, p, q, v1, v2, store);
+                        }
                     }
                     else
                     {
-                        l  = part * exp(fc[7] + coef - val1 * nd.q[f]);
-                        dl = l * (dcoef + val3 * nd.q[f]);
-                    }
-                    sL[e]  = l;
-                    sDl[e] = dl;
-                }
-                else if (tid >= SS && tid < SS + Dr)
-                {
-                    // corrected binding energy (net14.cpp:49-75) and screening mu/kT (:577-600)
-                    const int    s          = tid - SS;
-                    const double kbt        = phys::Kb * Tg;
-                    const double nakbt      = phys::Na * kbt;
-                    const double correction = -1.5 * nakbt;
-                    const double ne         = rho_t * phys::Na / 2.;
-                    {
-                        const double ae  = pow((3. / 4.) / (phys::pi * ne), 1. / 3.);
-                        const double gam = phys::e2 / (kbt * ae);
-                        const double gmm = gam * nd.Z53[s];
-                        const double fn  = gmm > 1 ? coulomb_strong(gmm) : coulomb_weak(gmm);
-                        double       be  = nd.BE0[s] + correction;
-                        be -= nakbt * fn;
-                        sBE[s] = be;
-                    }
-                    {
-                        const double kbt2 = Tg * phys::Kb;
-                        const double ae   = pow(3. / (4. * phys::pi * ne), 1. / 3.);
-                        const double gam  = phys::e2 / (kbt2 * ae);
-                        const double a1 = -.898004, b1 = .96786, c1 = .220703, d1 = -.86097, e1 = 2.520058332;
-                        const double gp  = gam * nd.Z53[s];
-                        const double sq  = sqrt(gp);
-                        const double sq2 = sqrt(sq);
-                        double       mu;
-                        if (gp <= 1)
-                            mu = -(1. / 1.7320508075688772) * gp * sq + pow(gp, 1.9885) * .29561 / 1.9885;
-                        else
-                            mu = a1 * gp + 4. * (b1 * sq2 - c1 / sq2) + d1 * log(gp) - e1;
-                        if (NET != 14 && s == 1) mu = 0; // neutron (net86.cpp:603)
-                        sMu[s] = mu;
-                    }
-                }
-                // hand-fitted rates.  net14: the groups' exp / pow values spread over the lanes of
-                // its one wavefront, then combined in every lane; net86 / net87: one group per lane
-                // on lanes of different wavefronts (measured faster there than the lane-parallel
-                // form on one of their wavefronts)
-                if constexpr (NET == 14)
-                {
-                    if ((tid >> 6) == 0)
-                    {
-                        // the values pass through the Jacobian array, which is rewritten only after
-                        // this phase: sJv[0 .. N1) level 1, sJv[N1 .. N1 + NE2) level 2
-                        static_assert(C::NNZ >= spx::N1 + spx::NE2, "hand-fitted values fit the Jacobian array");
-                        const int      k = tid & 63;
-                        const RatePow  p(Tg);
-                        const DerivPow q(Tg);
+                        // the t9 powers (functions of T alone) once per wavefront that holds a group,
+                        // in wave-uniform code, instead of once per group on its own lane
+                        static_assert(C::NT == 256, "groups on wavefronts 0-2 of four");
+                        if ((tid >> 6) < 3)
                         {
-                            const double t1 = special_level1(k, p, q);
-                            if (k < spx::N1) sJv[k] = t1;
-                        }
-                        psync<true>(); // one wavefront
-                        auto v1 = [&](int j) __attribute__((always_inline)) -> double { return sJv[j]; };
-                        {
-                            const double t2 = special_level2(k, p, q, v1);
-                            if (k < spx::NE2) sJv[spx::N1 + k] = t2;
-                        }
-                        psync<true>();
-                        auto v2 = [&](int j) __attribute__((always_inline)) -> double { return sJv[spx::N1 + j]; };
-                        // lane 0 stores each group's rate (and reverse) with its derivative
-                        auto store = [&](int g, double r, double rl, double dr, double drl) __attribute__((always_inline))
-                        {
-                            if (k != 0) return;
-                            const int e = g == 0 ? nd.sp.r3a_e : g == 1 ? nd.sp.r24 : g == 2 ? nd.sp.r1216 : g == 3 ? nd.sp.r32
-                                        : g == 4 ? nd.sp.rcag_e : nd.sp.roag_e;
-                            sEff[e]  = r;
-                            sDeff[e] = dr;
-                            if (g == 0 || g >= 4)
+                            const RatePow  p(Tg);
+                            const DerivPow q(Tg);
+                            const int g = special_task<NET>(tid);
+                            if (g >= 0)
                             {
-                                const int l = g == 0 ? nd.sp.r3a_l : g == 4 ? nd.sp.rcag_l : nd.sp.roag_l;
-                                sL[l]       = rl;
-                                sDl[l]      = drl;
-                            }
-                        };
-                        special_combine(Tg, p, q, v1, v2, store);
-                    }
-                }
-                else
-                {
-                    // the t9 powers (functions of T alone) once per wavefront that holds a group,
-                    // in wave-uniform code, instead of once per group on its own lane
-                    static_assert(C::NT == 256, "groups on wavefronts 0-2 of four");
-                    if ((tid >> 6) < 3)
-                    {
-                        const RatePow  p(Tg);
-                        const DerivPow q(Tg);
-                        const int g = special_task<NET>(tid);
-                        if (g >= 0)
-                        {
-                            double r = 0, rl = 0, dr = 0, drl = 0;
-                            if (g == 0)
-                            {
-                                special_triple_alpha(Tg, p, q, r, rl, dr, drl);
-                                sEff[nd.sp.r3a_e] = r, sDeff[nd.sp.r3a_e] = dr, sL[nd.sp.r3a_l] = rl, sDl[nd.sp.r3a_l] = drl;
-                            }
-                            else if (g == 1)
-                            {
-                                special_c12c12(Tg, p, q, r, dr);
-                                sEff[nd.sp.r24] = r, sDeff[nd.sp.r24] = dr;
-                            }
-                            else if (g == 2)
-                            {
-                                special_c12o16(Tg, p, q, r, dr);
-                                sEff[nd.sp.r1216] = r, sDeff[nd.sp.r1216] = dr;
-                            }
-                            else if (g == 3)
-                            {
-                                special_o16o16(Tg, p, q, r, dr);
-                                sEff[nd.sp.r32] = r, sDeff[nd.sp.r32] = dr;
-                            }
-                            else if (g == 4)
-                            {
-                                special_c12ag(Tg, p, q, r, rl, dr, drl);
-                                sEff[nd.sp.rcag_e] = r, sDeff[nd.sp.rcag_e] = dr, sL[nd.sp.rcag_l] = rl,
-                                sDl[nd.sp.rcag_l] = drl;
-                            }
-                            else
-                            {
-                                special_o16ag(Tg, p, q, r, rl, dr, drl);
-                                sEff[nd.sp.roag_e] = r, sDeff[nd.sp.roag_e] = dr, sL[nd.sp.roag_l] = rl,
-                                sDl[nd.sp.roag_l] = drl;
+                                double r = 0, rl = 0, dr = 0, drl = 0;
+                                if (g == 0)
+                                {
+                                    special_triple_alpha(Tg, p, q, r, rl, dr, drl);
+                                    sEff[nd.sp.r3a_e] = r, sDeff[nd.sp.r3a_e] = dr, sL[nd.sp.r3a_l] = rl, sDl[nd.sp.r3a_l] = drl;
+                                }
+                                else if (g == 1)
+                                {
+                                    special_c12c12(Tg, p, q, r, dr);
+                                    sEff[nd.sp.r24] = r, sDeff[nd.sp.r24] = dr;
+                                }
+                                else if (g == 2)
+                                {
+                                    special_c12o16(Tg, p, q, r, dr);
+                                    sEff[nd.sp.r1216] = r, sDeff[nd.sp.r1216] = dr;
+                                }
+                                else if (g == 3)
+                                {
+                                    special_o16o16(Tg, p, q, r, dr);
+                                    sEff[nd.sp.r32] = r, sDeff[nd.sp.r32] = dr;
+                                }
+                                else if (g == 4)
+                                {
+                                    special_c12ag(Tg, p, q, r, rl, dr, drl);
+                                    sEff[nd.sp.rcag_e] = r, sDeff[nd.sp.rcag_e] = dr, sL[nd.sp.rcag_l] = rl,
+                                    sDl[nd.sp.rcag_l] = drl;
+                                }
+                                else
+                                {
+                                    special_o16ag(Tg, p, q, r, rl, dr, drl);
+                                    sEff[nd.sp.roag_e] = r, sDeff[nd.sp.roag_e] = dr, sL[nd.sp.roag_l] = rl,
+                                    sDl[nd.sp.roag_l] = drl;
+                                }
                             }
                         }
                     }
+                    if (NET == 87 && (tid >> 6) == 1) // wavefront 1 (fitted rates, groups 2 and 5)
+                        electron_interpolate_wave(nd.elogT, nd.elogR, nd.etab, Tg, sYb[86] * rho_t, sEv, tid & 63);
+                    if (NET != 14 && tid == 225) sEff[3] = sDeff[3] = sL[3] = sDl[3] = 0; // unused slots
                 }
-                if (NET == 87 && (tid >> 6) == 1) // wavefront 1 (fitted rates, groups 2 and 5)
-                    electron_interpolate_wave(nd.elogT, nd.elogR, nd.etab, Tg, sYb[86] * rho_t, sEv, tid & 63);
-                if (NET != 14 && tid == 225) sEff[3] = sDeff[3] = sL[3] = sDl[3] = 0; // unused slots
-            }
-            psync<WAVE>();
+                psync<WAVE>();
 
-            // ---- rates, phase 2: swap, screening, reaction-list order ----
-            {
-                const double Tg = T_theta;
-                if (tid < nd.nE)
+                // ---- rates, phase 2: swap, screening, reaction-list order ----
                 {
-                    const int i = tid;
-                    double    e = sEff[i], de = sDeff[i], l = sL[i], dl = sDl[i];
-                    if (nd.swap[i])
+                    const double Tg = T_theta;
+                    if (tid < nd.nE)
                     {
-                        double t = e;
-                        e        = l;
-                        l        = t;
-                        t        = de;
-                        de       = dl;
-                        dl       = t;
+                        const int i = tid;
+                        double    e = sEff[i], de = sDeff[i], l = sL[i], dl = sDl[i];
+                        if (nd.swap[i])
+                        {
+                            double t = e;
+                            e        = l;
+                            l        = t;
+                            t        = de;
+                            de       = dl;
+                            dl       = t;
+                        }
+                        const int* sc = nd.scr + 4 * i;
+                        double     dm = sMu[sc[0]] + sMu[sc[1]] - sMu[sc[2]];
+                        // the optional fourth species (-1: none) is loaded through a selected index,
+                        // so a load issued ahead of the test still addresses sMu
+                        const double mu3 = sMu[sc[3] >= 0 ? sc[3] : 0];
+                        if (sc[3] >= 0) dm += mu3;
+                        const double EF = exp(dm);
+                        e               = e * EF;
+                        de              = de * EF - 2. * e * dm / Tg;
+                        if (nd.scr_l[i])
+                        {
+                            l  = l * EF;
+                            dl = dl * EF - 2. * l * dm / Tg;
+                        }
+                        if (nd.push_e[i] >= 0) sRate[nd.push_e[i]] = e, sDrt[nd.push_e[i]] = de;
+                        if (nd.push_l[i] >= 0) sRate[nd.push_l[i]] = l, sDrt[nd.push_l[i]] = dl;
                     }
-                    const int* sc = nd.scr + 4 * i;
-                    double     dm = sMu[sc[0]] + sMu[sc[1]] - sMu[sc[2]];
-                    // the optional fourth species (-1: none) is loaded through a selected index,
-                    // so a load issued ahead of the test still addresses sMu
-                    const double mu3 = sMu[sc[3] >= 0 ? sc[3] : 0];
-                    if (sc[3] >= 0) dm += mu3;
-                    const double EF = exp(dm);
-                    e               = e * EF;
-                    de              = de * EF - 2. * e * dm / Tg;
-                    if (nd.scr_l[i])
+                    if (NET == 87 && tid == NT - 1)
                     {
-                        l  = l * EF;
-                        dl = dl * EF - 2. * l * dm / Tg;
+                        // net87.hpp:153-174
+                        const double kbt        = phys::Kb * Tg;
+                        const double nakbt      = phys::Na * kbt;
+                        const double correction = -1.5 * nakbt;
+                        sBE[86]                 = nd.BEe + correction;
+                        sBE[0] += -sEv[3];
+                        sBE[1] += -sEv[9];
+                        const double rhoElec = sYb[86] * rho_t;
+                        sRate[309]           = rhoElec == 0 ? 0 : sEv[0] / rhoElec;
+                        sDrt[309]            = rhoElec == 0 ? 0 : sEv[1] / rhoElec;
+                        sRate[310]           = rhoElec == 0 ? 0 : sEv[6] / rhoElec;
+                        sDrt[310]            = rhoElec == 0 ? 0 : sEv[7] / rhoElec;
                     }
-                    if (nd.push_e[i] >= 0) sRate[nd.push_e[i]] = e, sDrt[nd.push_e[i]] = de;
-                    if (nd.push_l[i] >= 0) sRate[nd.push_l[i]] = l, sDrt[nd.push_l[i]] = dl;
                 }
-                if (NET == 87 && tid == NT - 1)
-                {
-                    // net87.hpp:153-174
-                    const double kbt        = phys::Kb * Tg;
-                    const double nakbt      = phys::Na * kbt;
-                    const double correction = -1.5 * nakbt;
-                    sBE[86]                 = nd.BEe + correction;
-                    sBE[0] += -sEv[3];
-                    sBE[1] += -sEv[9];
-                    const double rhoElec = sYb[86] * rho_t;
-                    sRate[309]           = rhoElec == 0 ? 0 : sEv[0] / rhoElec;
-                    sDrt[309]            = rhoElec == 0 ? 0 : sEv[1] / rhoElec;
-                    sRate[310]           = rhoElec == 0 ? 0 : sEv[6] / rhoElec;
-                    sDrt[310]            = rhoElec == 0 ? 0 : sEv[7] / rhoElec;
-                }
-            }
-            psync<WAVE>();
+                psync<WAVE>();
 
-            // ---- per-reaction mass-action factors (nuclear_net.hpp:355-371, 404-426) ----
-            // slot s computes reaction maperm[s]: the wavefronts that run a second pass take the
-            // cheapest reactions
-            for (int s = tid; s < nd.nR; s += NT)
-            {
-                const int    r = maperm[s];
-                double       v = sRate[r], dv = sDrt[r], jr = sRate[r];
-                const int    q0 = rx[r] & 0xffff, q1 = rx[r] >> 16;
-                for (int q = q0; q < q1; ++q)
+                // ---- per-reaction mass-action factors (nuclear_net.hpp:355-371, 404-426) ----
+                // slot s computes reaction maperm[s]: the wavefronts that run a second pass take the
+                // cheapest reactions
+                for (int s = tid; s < nd.nR; s += NT)
                 {
-                    const int    c = ent16[q] >> 8;
-                    const double x = sYb[ent16[q] & 0xff] * rho_t;
-                    if (c != 1)
+                    const int    r = maperm[s];
+                    double       v = sRate[r], dv = sDrt[r], jr = sRate[r];
+                    const int    q0 = rx[r] & 0xffff, q1 = rx[r] >> 16;
+                    for (int q = q0; q < q1; ++q)
                     {
-                        const double fct = factorial_count(c);
-                        v                = v / fct;
-                        dv               = dv / fct;
-                        jr               = jr / fct;
+                        const int    c = ent16[q] >> 8;
+                        const double x = sYb[ent16[q] & 0xff] * rho_t;
+                        if (c != 1)
+                        {
+                            const double fct = factorial_count(c);
+                            v                = v / fct;
+                            dv               = dv / fct;
+                            jr               = jr / fct;
+                        }
+                        v  = v * pow_count(x, c);
+                        dv = dv * pow_count(x, c);
+                        jr = jr * pow_count(x, c - 1);
                     }
-                    v  = v * pow_count(x, c);
-                    dv = dv * pow_count(x, c);
-                    jr = jr * pow_count(x, c - 1);
+                    sVal[r]       = v / rho_t;
+                    sDval[r]      = dv / rho_t;
+                    const bool ok = jr > k::epsilonSystem;
+                    sJok[r]       = ok ? 1. : 0.;
+                    if (ok)
+                        for (int qa = q0; qa < q1; ++qa)
+                        {
+                            const int b   = ent16[qa] & 0xff;
+                            double    tr_ = jr;
+                            for (int o = q0; o < q1; ++o)
+                                if ((ent16[o] & 0xff) != b) tr_ *= sYb[ent16[o] & 0xff] * rho_t;
+                            sTr[r * MAXQ + (qa - q0)] = tr_;
+                        }
                 }
-                sVal[r]       = v / rho_t;
-                sDval[r]      = dv / rho_t;
-                const bool ok = jr > k::epsilonSystem;
-                sJok[r]       = ok ? 1. : 0.;
-                if (ok)
-                    for (int qa = q0; qa < q1; ++qa)
-                    {
-                        const int b   = ent16[qa] & 0xff;
-                        double    tr_ = jr;
-                        for (int o = q0; o < q1; ++o)
-                            if ((ent16[o] & 0xff) != b) tr_ *= sYb[ent16[o] & 0xff] * rho_t;
-                        sTr[r * MAXQ + (qa - q0)] = tr_;
-                    }
-            }
-            psync<WAVE>();
+                psync<WAVE>();
 
-            // ---- Jacobian non-zeros (firstOrderDYFromReactions) and species sums
-            //      (derivativesFromReactions), each summed in the reference's order ----
-            // non-zeros are handed out in descending order of their list lengths, so the lanes of
-            // one pass over the workgroup have lists of similar length (lane-to-slot map: jac_slot)
-            for (int pass = 0;; ++pass)
-            {
-                const int k = jac_slot(tid, pass, NT, nd.nnz);
-                if (k >= nd.nnz) break;
-                const int e = jord16[k];
-                // J = sum over the entry's contributions in list order of count * mass-action
-                // derivative, skipping reactions whose derivative factor is <= 1e-40; eight
-                // contributions are loaded ahead of their (sequential) additions
-                double    J  = 0.;
-                int       kk = nzp16[e];
-                const int k1 = nzp16[e + 1];
-                for (; kk + 8 <= k1; kk += 8)
+                // ---- Jacobian non-zeros (firstOrderDYFromReactions) and species sums
+                //      (derivativesFromReactions), each summed in the reference's order ----
+                // non-zeros are handed out in descending order of their list lengths, so the lanes of
+                // one pass over the workgroup have lists of similar length (lane-to-slot map: jac_slot)
+                for (int pass = 0;; ++pass)
                 {
-                    // stage 1: the eight entry words; stage 2: their factors; then the additions
-                    // (scheduling barriers keep each stage's loads in flight together)
-                    uint32_t w[8];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u)
-                        w[u] = nzent[kk + u];
-                    __builtin_amdgcn_sched_barrier(0);
-                    double tr[8], okv[8];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u)
+                    const int k = jac_slot(tid, pass, NT, nd.nnz);
+                    if (k >= nd.nnz) break;
+                    const int e = jord16[k];
+                    // J = sum over the entry's contributions in list order of count * mass-action
+                    // derivative, skipping reactions whose derivative factor is <= 1e-40; eight
+                    // contributions are loaded ahead of their (sequential) additions
+                    double    J  = 0.;
+                    int       kk = nzp16[e];
+                    const int k1 = nzp16[e + 1];
+                    for (; kk + 8 <= k1; kk += 8)
                     {
-                        const int r = w[u] & 0xfff;
-                        okv[u]      = sJok[r];
-                        tr[u]       = sTr[r * MAXQ + ((w[u] >> 12) & 0xf)];
+                        // stage 1: the eight entry words; stage 2: their factors; then the additions
+                        // (scheduling barriers keep each stage's loads in flight together)
+                        uint32_t w[8];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                            w[u] = nzent[kk + u];
+                        __builtin_amdgcn_sched_barrier(0);
+                        double tr[8], okv[8];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                        {
+                            const int r = w[u] & 0xfff;
+                            okv[u]      = sJok[r];
+                            tr[u]       = sTr[r * MAXQ + ((w[u] >> 12) & 0xf)];
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                        {
+                            const double t = tr[u] * (double)(int8_t)(w[u] >> 16);
+                            J              = okv[u] != 0. ? J + t : J;
+                        }
                     }
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int u = 0; u < 8; ++u)
+                    for (; kk < k1; ++kk)
                     {
-                        const double t = tr[u] * (double)(int8_t)(w[u] >> 16);
-                        J              = okv[u] != 0. ? J + t : J;
+                        const uint32_t w  = nzent[kk];
+                        const int      r  = w & 0xfff;
+                        const double   t  = sTr[r * MAXQ + ((w >> 12) & 0xf)] * (double)(int8_t)(w >> 16);
+                        J                 = sJok[r] != 0. ? J + t : J;
+                    }
+                    sJv[e] = J;
+                }
+                // dY/dt and d(dY/dt)/dT per species: signed-count sums in list order.  Nothing reads
+                // them before the matrix fill, so with several wavefronts per particle each sum takes
+                // its first KPRE entries here and the rest after the barrier, beside the RHS
+                // correction of the other lanes (the longest species lists -- 140 entries for two
+                // net86 species -- would otherwise hold every wavefront at the barrier); one
+                // wavefront has nothing to overlap.  The additions keep their order across the split.
+                constexpr bool SPLIT = C::NT > 64;
+                constexpr int  KPRE  = SPLIT ? 72 : 1 << 20; // 72 measured faster than 96 on net86
+                static_assert(2 * D <= NT, "species lanes [NT - D, NT) and RHS lanes [0, D) are disjoint");
+                const int     sps  = tid - (NT - D);
+                double        spa = 0., spb = 0.;
+                int           spe = 0, spe1 = 0;
+                auto species_sum = [&](int e1) __attribute__((always_inline))
+                {
+                    int e = spe;
+                    for (; e + 8 <= e1; e += 8)
+                    {
+                        uint32_t w[8];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                            w[u] = spent[e + u];
+                        __builtin_amdgcn_sched_barrier(0);
+                        double x[8], y[8];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                        {
+                            const int r = w[u] & 0xffff;
+                            x[u]        = sVal[r];
+                            y[u]        = sDval[r];
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                        {
+                            const double c = (double)(int8_t)(w[u] >> 16);
+                            spa            = spa + x[u] * c;
+                            spb            = spb + y[u] * c;
+                        }
+                    }
+                    for (; e < e1; ++e)
+                    {
+                        const uint32_t w = spent[e];
+                        const int      r = w & 0xffff;
+                        const double   c = (double)(int8_t)(w >> 16);
+                        spa              = spa + sVal[r] * c;
+                        spb              = spb + sDval[r] * c;
+                    }
+                    spe = e;
+                };
+                // Yg - Y per species for the RHS correction, into the screening array (dead after the
+                // rate phase): the difference the reference forms inside that sum, formed once here
+                double* sDYg = sMu;
+                if (sps >= 0)
+                {
+                    sDYg[sps] = sYb[sps] - sY[sps];
+                    spe  = spp16[sps];
+                    spe1 = spp16[sps + 1];
+                    species_sum(spe1 - spe > KPRE ? spe + KPRE : spe1);
+                    if constexpr (!SPLIT)
+                    {
+                        sDYd[sps] = spa;
+                        sDYT[sps] = spb;
                     }
                 }
-                for (; kk < k1; ++kk)
+                psync<WAVE>();
+                // RHS correction sum_j J[a][j] (Yg[j] - Y[j]) over the row's non-zeros, j ascending
+                if (tid < D)
                 {
-                    const uint32_t w  = nzent[kk];
-                    const int      r  = w & 0xfff;
-                    const double   t  = sTr[r * MAXQ + ((w >> 12) & 0xf)] * (double)(int8_t)(w >> 16);
-                    J                 = sJok[r] != 0. ? J + t : J;
-                }
-                sJv[e] = J;
-            }
-            // dY/dt and d(dY/dt)/dT per species: signed-count sums in list order.  Nothing reads
-            // them before the matrix fill, so with several wavefronts per particle each sum takes
-            // its first KPRE entries here and the rest after the barrier, beside the RHS
-            // correction of the other lanes (the longest species lists -- 140 entries for two
-            // net86 species -- would otherwise hold every wavefront at the barrier); one
-            // wavefront has nothing to overlap.  The additions keep their order across the split.
-            constexpr bool SPLIT = C::NT > 64;
-            constexpr int  KPRE  = SPLIT ? 72 : 1 << 20; // 72 measured faster than 96 on net86
-            static_assert(2 * D <= NT, "species lanes [NT - D, NT) and RHS lanes [0, D) are disjoint");
-            const int     sps  = tid - (NT - D);
-            double        spa = 0., spb = 0.;
-            int           spe = 0, spe1 = 0;
-            auto species_sum = [&](int e1) __attribute__((always_inline))
-            {
-                int e = spe;
-                for (; e + 8 <= e1; e += 8)
-                {
-                    uint32_t w[8];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u)
-                        w[u] = spent[e + u];
-                    __builtin_amdgcn_sched_barrier(0);
-                    double x[8], y[8];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u)
+                    double    corr = 0;
+                    int       e    = rowp16[tid];
+                    const int e1   = rowp16[tid + 1];
+                    for (; e + 8 <= e1; e += 8)
                     {
-                        const int r = w[u] & 0xffff;
-                        x[u]        = sVal[r];
-                        y[u]        = sDval[r];
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
+                        uint32_t w[8];
 #pragma unroll
-                    for (int u = 0; u < 8; ++u)
-                    {
-                        const double c = (double)(int8_t)(w[u] >> 16);
-                        spa            = spa + x[u] * c;
-                        spb            = spb + y[u] * c;
+                        for (int u = 0; u < 8; ++u)
+                            w[u] = rowent[e + u];
+                        __builtin_amdgcn_sched_barrier(0);
+                        double jv[8], dy[8];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                        {
+                            jv[u] = sJv[w[u] & 0xffff];
+                            dy[u] = sDYg[w[u] >> 16];
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                            corr = corr + jv[u] * dy[u];
                     }
+                    for (; e < e1; ++e)
+                    {
+                        const uint32_t w = rowent[e];
+                        corr             = corr + sJv[w & 0xffff] * sDYg[w >> 16];
+                    }
+                    sCorr[tid] = corr;
                 }
-                for (; e < e1; ++e)
+                else if (SPLIT && sps >= 0)
                 {
-                    const uint32_t w = spent[e];
-                    const int      r = w & 0xffff;
-                    const double   c = (double)(int8_t)(w >> 16);
-                    spa              = spa + sVal[r] * c;
-                    spb              = spb + sDval[r] * c;
-                }
-                spe = e;
-            };
-            // Yg - Y per species for the RHS correction, into the screening array (dead after the
-            // rate phase): the difference the reference forms inside that sum, formed once here
-            double* sDYg = sMu;
-            if (sps >= 0)
-            {
-                sDYg[sps] = sYb[sps] - sY[sps];
-                spe  = spp16[sps];
-                spe1 = spp16[sps + 1];
-                species_sum(spe1 - spe > KPRE ? spe + KPRE : spe1);
-                if constexpr (!SPLIT)
-                {
+                    species_sum(spe1);
                     sDYd[sps] = spa;
                     sDYT[sps] = spb;
                 }
+                psync<WAVE>();
             }
-            // this lane's register-slot mask and first non-zero id (for the matrix fill)
-            const uint4 lmap = nd.lanemap[tid];
-            psync<WAVE>();
-            // RHS correction sum_j J[a][j] (Yg[j] - Y[j]) over the row's non-zeros, j ascending
-            if (tid < D)
-            {
-                double    corr = 0;
-                int       e    = rowp16[tid];
-                const int e1   = rowp16[tid + 1];
-                for (; e + 8 <= e1; e += 8)
-                {
-                    uint32_t w[8];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u)
-                        w[u] = rowent[e + u];
-                    __builtin_amdgcn_sched_barrier(0);
-                    double jv[8], dy[8];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u)
-                    {
-                        jv[u] = sJv[w[u] & 0xffff];
-                        dy[u] = sDYg[w[u] >> 16];
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int u = 0; u < 8; ++u)
-                        corr = corr + jv[u] * dy[u];
-                }
-                for (; e < e1; ++e)
-                {
-                    const uint32_t w = rowent[e];
-                    corr             = corr + sJv[w & 0xffff] * sDYg[w >> 16];
-                }
-                sCorr[tid] = corr;
-            }
-            else if (SPLIT && sps >= 0)
-            {
-                species_sum(spe1);
-                sDYd[sps] = spa;
-                sDYT[sps] = spb;
-            }
-            psync<WAVE>();
 
             // ---- Newton matrix into registers (nuclear_net.hpp:551-608) ----
             double cvv, dpdTv;
@@ -1742,6 +1756,7 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
                 elapsed += timestep;
                 ++n_sub;
                 cyc.lim = 0;
+                kept    = false;
                 if ((dt_tot - elapsed) / dt_tot < k::substep_dtTol) break;
             }
             else if (i == 0)
