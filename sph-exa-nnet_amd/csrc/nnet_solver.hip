@@ -991,6 +991,11 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
             const bool  again = kept && i == 1;
             const uint4 lmap  = nd.lanemap[tid]; // register-slot mask, first non-zero id (matrix fill)
             kept              = i == 1;
+            // an opaque lane index (range restored): the lane's addresses are formed in each iteration,
+            // not kept from the kernel's entry and spilled (net86 Helmholtz FP64: 67 -> 19 VGPRs, net14
+            // 137 -> 84; 524,288 net86 particles 568 -> 536 ms, 4,099 of net87 at cap 2,000 95 -> 87 ms)
+            asm volatile("" : "+v"(tid));
+            tid &= NT - 1;
             if (!again)
             {
                 for (int s = tid; s < D; s += NT)
