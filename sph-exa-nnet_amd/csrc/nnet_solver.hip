@@ -835,19 +835,6 @@ struct PanelLU
     }
 };
 
-// Hand-fitted rate group computed by lane tid (-1: none).
-template<int NET>
-__device__ __forceinline__ int special_task(int tid)
-{
-    // net86/net87: groups 0, 1 and 3 on wavefront 0 and groups 2 and 5 on wavefront 1 (next to
-    // the fitted rates; net87's electron captures also run on wavefront 1), group 4 on wavefront 2
-    // (fitted rates + species); wavefront 3 runs the species and the EOS lane.  These placements
-    // measured the shortest rate phase (its slowest wavefront sets its length).
-    if (NET == 86) return (tid == 32 || tid == 33) ? tid - 32 : tid == 96 ? 2 : tid == 34 ? 3 : tid == 160 ? 4 : tid == 98 ? 5 : -1;
-    if (NET == 87) return (tid == 32 || tid == 33) ? tid - 32 : tid == 96 ? 2 : tid == 34 ? 3 : tid == 160 ? 4 : tid == 99 ? 5 : -1;
-    return -1; // net14: the lane-parallel form on its one wavefront
-}
-
 // ---------------------------------------------------------------------------------------------
 // The solve: the Cfg<NET>::NT lanes of one particle group take particles from the batch's work
 // queue and integrate each over one hydro step, until the queue is empty.  sm: the group's
@@ -1041,172 +1028,120 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
                 }
                 {
                     const double Tg = T_theta;
-                    const int    SS = nd.nfit; // species lanes follow the fitted-rate lanes
-                    if (tid < nd.nfit)
+                    const int    k = tid & 63, w = NT == 64 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);
+                    // net14's one wavefront has the fitted rates' exps among the lanes of the groups' exp
+                    // pass: lane F0 + f the forward one of fitted rate f, F0 + nfit + f the reverse;
+                    // net86 / net87: lane f both, and the groups' pass of its own on wavefronts 0-2
+                    constexpr int F0  = spx::NE1 + spx::NE2;
+                    const int     f   = NET == 14 ? (k >= F0 + nd.nfit ? k - F0 - nd.nfit : k - F0) : tid;
+                    const bool    fit = f >= 0 && f < nd.nfit;
+                    // one pow and one log pass (pow_lane; log of the fitted rates' two forms of t9)
+                    const double pv  = pow_lane(k, Tg, rho_t);
+                    const double rt9 = nd.rev_div ? Tg / 1.e9 : Tg * 1e-09;
+                    double       ea = 0., el = 0., dcoef = 0., drev = 0., part = 0.;
+                    if (w < 3) // (the fitted rates of net86 / net87 end on wavefront 2)
                     {
-                        const int     f  = tid;
-                        const double* fc = nd.fit + 8 * f;
-                        const double  t9 = Tg / 1.e9, t913 = pow(t9, 1. / 3.), t923 = t913 * t913, t953 = pow(t9, 5. / 3.);
-                        const double  t9i = 1.e0 / t9, t9i2 = t9i * t9i, t9i13 = 1.e0 / t913, t9i23 = t9i13 * t9i13,
-                                     t9i43 = t9i23 * t9i23, lt9 = log(t9);
-                        const double coef =
-                            fc[1] * t9i + fc[2] * t9i13 + fc[3] * t913 + fc[4] * t9 + fc[5] * t953 + fc[6] * lt9;
-                        const double dcoef =
-                            (-fc[1] * t9i2 + (-fc[2] * t9i43 + fc[3] * t9i23 + 5 * fc[5] * t923) * (1. / 3.) + fc[4] +
-                             fc[6] * t9i) *
-                            1e-9;
-                        const int    e   = nd.fit_e0 + f;
-                        const double eff = exp(fc[0] + coef);
-                        sEff[e]          = eff;
-                        sDeff[e]         = eff * dcoef;
-                        // reverse rate (net14.cpp:150-190, net86.cpp:524-554)
-                        const double rt9  = nd.rev_div ? Tg / 1.e9 : Tg * 1e-09;
-                        const double rt9i = 1. / rt9;
-                        const double val1 = 11.6045 * rt9i;
-                        const double val3 = val1 * rt9i * 1e-9;
-                        const int    kb   = temperature_bin(Tg);
-                        const double part = nd.choose[nd.ca[f] * 24 + kb] / nd.choose[nd.cb[f] * 24 + kb];
-                        double       l, dl;
-                        if (nd.photo[f])
+                        const double t9 = Tg / 1.e9;
+                        const double lg = log(k == 1 ? rt9 : t9);
+                        const double lt9 = bcast_lane(lg, 0), lrt9 = bcast_lane(lg, 1);
+                        const double t913 = bcast_lane(pv, spx::PF13), t953 = bcast_lane(pv, spx::PF53);
+                        if (fit)
                         {
-                            const double val2 = 1.5 * log(rt9);
-                            const double val4 = 1.5e-9 * rt9i;
-                            l                 = part * exp(fc[7] + coef - val1 * nd.q[f] + val2);
-                            dl                = l * (dcoef + val3 * nd.q[f] + val4);
+                            const double* fc = nd.fit + 8 * f;
+                            const double  t923 = t913 * t913;
+                            const double  t9i = 1.e0 / t9, t9i2 = t9i * t9i, t9i13 = 1.e0 / t913, t9i23 = t9i13 * t9i13,
+                                         t9i43 = t9i23 * t9i23;
+                            const double coef =
+                                fc[1] * t9i + fc[2] * t9i13 + fc[3] * t913 + fc[4] * t9 + fc[5] * t953 + fc[6] * lt9;
+                            dcoef = (-fc[1] * t9i2 + (-fc[2] * t9i43 + fc[3] * t9i23 + 5 * fc[5] * t923) * (1. / 3.) +
+                                     fc[4] + fc[6] * t9i) *
+                                    1e-9;
+                            // reverse rate (net14.cpp:150-190, net86.cpp:524-554)
+                            const double rt9i = 1. / rt9;
+                            const double val1 = 11.6045 * rt9i;
+                            const double val3 = val1 * rt9i * 1e-9;
+                            const int    kb   = temperature_bin(Tg);
+                            part              = nd.choose[nd.ca[f] * 24 + kb] / nd.choose[nd.cb[f] * 24 + kb];
+                            const double qf   = nd.q[f];
+                            ea                = fc[0] + coef;
+                            el                = fc[7] + coef - val1 * qf;
+                            drev              = dcoef + val3 * qf;
+                            if (nd.photo[f])
+                            {
+                                el   = el + 1.5 * lrt9;
+                                drev = drev + 1.5e-9 * rt9i;
+                            }
                         }
-                        else
-                        {
-                            l  = part * exp(fc[7] + coef - val1 * nd.q[f]);
-                            dl = l * (dcoef + val3 * nd.q[f]);
-                        }
-                        sL[e]  = l;
-                        sDl[e] = dl;
                     }
-                    else if (tid >= SS && tid < SS + Dr)
+                    auto forward = [&](double eff) __attribute__((always_inline))
                     {
-                        // corrected binding energy (net14.cpp:49-75) and screening mu/kT (:577-600)
-                        const int    s          = tid - SS;
-                        const double kbt        = phys::Kb * Tg;
-                        const double nakbt      = phys::Na * kbt;
-                        const double correction = -1.5 * nakbt;
-                        const double ne         = rho_t * phys::Na / 2.;
+                        const int e = nd.fit_e0 + f;
+                        sEff[e]     = eff;
+                        sDeff[e]    = eff * dcoef;
+                    };
+                    auto reverse = [&](double er) __attribute__((always_inline))
+                    {
+                        const int    e = nd.fit_e0 + f;
+                        const double l = part * er;
+                        sL[e]          = l;
+                        sDl[e]         = l * drev;
+                    };
+                    if (NET != 14 && fit)
+                    {
+                        forward(exp(ea));
+                        reverse(exp(el));
+                    }
+                    // species lanes: net14 the first lanes, net86 / net87 those after the fitted rates'
+                    const int s = NET == 14 ? k : tid - nd.nfit;
+                    if (s >= 0 && s < Dr)
+                    {
+                        double be, mu;
+                        species_coulomb(Tg, bcast_lane(pv, spx::PAE), nd.Z53[s], nd.BE0[s], be, mu);
+                        if (NET != 14 && s == 1) mu = 0; // neutron (net86.cpp:603)
+                        sBE[s] = be;
+                        sMu[s] = mu;
+                    }
+                    // hand-fitted groups
+                    if (w < 3)
+                    {
+                        const RatePow  p(Tg, bcast_lane(pv, spx::PR13));
+                        const DerivPow q(Tg, bcast_lane(pv, spx::PD13));
+                        double         a = exp_arg(spx_arg[k], p, q, pv);
+                        if (NET == 14 && fit) a = k >= F0 + nd.nfit ? el : ea;
+                        const double ev = exp(a);
+                        if (NET == 14 && fit)
                         {
-                            const double ae  = pow((3. / 4.) / (phys::pi * ne), 1. / 3.);
-                            const double gam = phys::e2 / (kbt * ae);
-                            const double gmm = gam * nd.Z53[s];
-                            const double fn  = gmm > 1 ? coulomb_strong(gmm) : coulomb_weak(gmm);
-                            double       be  = nd.BE0[s] + correction;
-                            be -= nakbt * fn;
-                            sBE[s] = be;
-                        }
-                        {
-                            const double kbt2 = Tg * phys::Kb;
-                            const double ae   = pow(3. / (4. * phys::pi * ne), 1. / 3.);
-                            const double gam  = phys::e2 / (kbt2 * ae);
-                            const double a1 = -.898004, b1 = .96786, c1 = .220703, d1 = -.86097, e1 = 2.520058332;
-                            const double gp  = gam * nd.Z53[s];
-                            const double sq  = sqrt(gp);
-                            const double sq2 = sqrt(sq);
-                            double       mu;
-                            if (gp <= 1)
-                                mu = -(1. / 1.7320508075688772) * gp * sq + pow(gp, 1.9885) * .29561 / 1.9885;
+                            if (k >= F0 + nd.nfit)
+                                reverse(ev);
                             else
-                                mu = a1 * gp + 4. * (b1 * sq2 - c1 / sq2) + d1 * log(gp) - e1;
-                            if (NET != 14 && s == 1) mu = 0; // neutron (net86.cpp:603)
-                            sMu[s] = mu;
+                                forward(ev);
                         }
-                    }
-                    // hand-fitted rates.  net14: the groups' exp / pow values spread over the lanes of
-                    // its one wavefront, then combined in every lane; net86 / net87: one group per lane
-                    // on lanes of different wavefronts (measured faster there than the lane-parallel
-                    // form on one of their wavefronts)
-                    if constexpr (NET == 14)
-                    {
-                        if ((tid >> 6) == 0)
+                        auto v1 = [&](int j) __attribute__((always_inline)) -> double
+                        { return j < spx::NE1 ? bcast_lane(ev, j) : bcast_lane(pv, spx::PL1 + j - spx::NE1); };
+                        auto v2 = [&](int j) __attribute__((always_inline)) -> double { return bcast_lane(ev, spx::NE1 + j); };
+                        // lane 0 stores each group's rate (and reverse) with its derivative
+                        auto store = [&](int g, double r, double rl, double dr, double drl) __attribute__((always_inline))
                         {
-                            // the values pass through the Jacobian array, which is rewritten only after
-                            // this phase: sJv[0 .. N1) level 1, sJv[N1 .. N1 + NE2) level 2
-                            static_assert(C::NNZ >= spx::N1 + spx::NE2, "hand-fitted values fit the Jacobian array");
-                            const int      k = tid & 63;
-                            const RatePow  p(Tg);
-                            const DerivPow q(Tg);
+                            if (k != 0) return;
+                            const int e = g == 0 ? nd.sp.r3a_e : g == 1 ? nd.sp.r24 : g == 2 ? nd.sp.r1216 : g == 3 ? nd.sp.r32
+                                        : g == 4 ? nd.sp.rcag_e : nd.sp.roag_e;
+                            sEff[e]  = r;
+                            sDeff[e] = dr;
+                            if (g == 0 || g >= 4)
                             {
-                                const double t1 = special_level1(k, p, q);
-                                if (k < spx::N1) sJv[k] = t1;
+                                const int l = g == 0 ? nd.sp.r3a_l : g == 4 ? nd.sp.rcag_l : nd.sp.roag_l;
+                                sL[l]       = rl;
+                                sDl[l]      = drl;
                             }
-                            psync<true>(); // one wavefront
-                            auto v1 = [&](int j) __attribute__((always_inline)) -> double { return sJv[j]; };
-                            {
-                                const double t2 = special_level2(k, p, q, v1);
-                                if (k < spx::NE2) sJv[spx::N1 + k] = t2;
-                            }
-                            psync<true>();
-                            auto v2 = [&](int j) __attribute__((always_inline)) -> double { return sJv[spx::N1 + j]; };
-                            // lane 0 stores each group's rate (and reverse) with its derivative
-                            auto store = [&](int g, double r, double rl, double dr, double drl) __attribute__((always_inline))
-                            {
-                                if (k != 0) return;
-                                const int e = g == 0 ? nd.sp.r3a_e : g == 1 ? nd.sp.r24 : g == 2 ? nd.sp.r1216 : g == 3 ? nd.sp.r32
-                                            : g == 4 ? nd.sp.rcag_e : nd.sp.roag_e;
-                                sEff[e]  = r;
-                                sDeff[e] = dr;
-                                if (g == 0 || g >= 4)
-                                {
-                                    const int l = g == 0 ? nd.sp.r3a_l : g == 4 ? nd.sp.rcag_l : nd.sp.roag_l;
-                                    sL[l]       = rl;
-                                    sDl[l]      = drl;
-                                }
-                            };
-                            special_combine(Tg, p, q, v1, v2, store);
-                        }
-                    }
-                    else
-                    {
-                        // the t9 powers (functions of T alone) once per wavefront that holds a group,
-                        // in wave-uniform code, instead of once per group on its own lane
-                        static_assert(C::NT == 256, "groups on wavefronts 0-2 of four");
-                        if ((tid >> 6) < 3)
-                        {
-                            const RatePow  p(Tg);
-                            const DerivPow q(Tg);
-                            const int g = special_task<NET>(tid);
-                            if (g >= 0)
-                            {
-                                double r = 0, rl = 0, dr = 0, drl = 0;
-                                if (g == 0)
-                                {
-                                    special_triple_alpha(Tg, p, q, r, rl, dr, drl);
-                                    sEff[nd.sp.r3a_e] = r, sDeff[nd.sp.r3a_e] = dr, sL[nd.sp.r3a_l] = rl, sDl[nd.sp.r3a_l] = drl;
-                                }
-                                else if (g == 1)
-                                {
-                                    special_c12c12(Tg, p, q, r, dr);
-                                    sEff[nd.sp.r24] = r, sDeff[nd.sp.r24] = dr;
-                                }
-                                else if (g == 2)
-                                {
-                                    special_c12o16(Tg, p, q, r, dr);
-                                    sEff[nd.sp.r1216] = r, sDeff[nd.sp.r1216] = dr;
-                                }
-                                else if (g == 3)
-                                {
-                                    special_o16o16(Tg, p, q, r, dr);
-                                    sEff[nd.sp.r32] = r, sDeff[nd.sp.r32] = dr;
-                                }
-                                else if (g == 4)
-                                {
-                                    special_c12ag(Tg, p, q, r, rl, dr, drl);
-                                    sEff[nd.sp.rcag_e] = r, sDeff[nd.sp.rcag_e] = dr, sL[nd.sp.rcag_l] = rl,
-                                    sDl[nd.sp.rcag_l] = drl;
-                                }
-                                else
-                                {
-                                    special_o16ag(Tg, p, q, r, rl, dr, drl);
-                                    sEff[nd.sp.roag_e] = r, sDeff[nd.sp.roag_e] = dr, sL[nd.sp.roag_l] = rl,
-                                    sDl[nd.sp.roag_l] = drl;
-                                }
-                            }
-                        }
+                        };
+                        if (NET == 14)
+                            special_combine<63>(Tg, p, q, v1, v2, store);
+                        else if (w == 0)
+                            special_combine<9>(Tg, p, q, v1, v2, store);
+                        else if (w == 1)
+                            special_combine<6>(Tg, p, q, v1, v2, store);
+                        else
+                            special_combine<48>(Tg, p, q, v1, v2, store);
                     }
                     if (NET == 87 && (tid >> 6) == 1) // wavefront 1 (fitted rates, groups 2 and 5)
                         electron_interpolate_wave(nd.elogT, nd.elogR, nd.etab, Tg, sYb[86] * rho_t, sEv, tid & 63);
