@@ -947,7 +947,12 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
         bool         abandon = false; // mixed pass: FP32 refinement failed, left to the FP64 redo pass
         uint8_t      status = NNET_STATUS_OK;
         cyc.lim             = 0;
-        bool         kept = false; // the assembly arrays are those of the accepted state
+        // the assembly arrays of the accepted state (what the matrix fill reads of them): not computed,
+        // in LDS, or kept in registers while LDS holds those of a later iteration
+        enum { NONE, IN_LDS, IN_REG };
+        constexpr int KEEP = L::phaseEnd - L::oBE, NKEEP = (KEEP + NT - 1) / NT;
+        int           kept = NONE;
+        double        keep[NKEEP] = {};
 
         for (int i = 1;; ++i)
         {
@@ -970,14 +975,29 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
             const double T_theta = (1 - k::theta) * T + k::theta * T_loc;
             // A rejected attempt restarts from the accepted state, and its first iteration linearises
             // there whatever its timestep: rates, EOS, Jacobian and their sums are those of the attempt
-            // before it, still in the assembly arrays when that one was rejected in its first iteration
-            // too (a later iteration or another state has written them otherwise).  Such an iteration
-            // is the matrix fill and the solve alone, and most iterations of a capped particle are of
-            // this kind.  50,021 net14 particles, first step: 533 -> 84 ms; 4,099 of net87, whose
-            // attempts mostly fail later: unchanged (93 ms).
-            const bool  again = kept && i == 1;
+            // before it.  They are still in the assembly arrays when that one was rejected in its first
+            // iteration too; before a later iteration writes those arrays, each lane keeps its share of
+            // what the fill reads.  Such a first iteration is the matrix fill and the solve alone, and
+            // most iterations of a capped particle are of this kind.  50,021 net14 particles, first step:
+            // 533 -> 84 ms; 4,099 of net87 at cap 2,000, whose attempts fail in their second
+            // to fourth iteration: 79.4 -> 71.8 ms.
             const uint4 lmap  = nd.lanemap[tid]; // register-slot mask, first non-zero id (matrix fill)
-            kept              = i == 1;
+            const bool  again = i == 1 && kept != NONE;
+            if (i > 1 && kept == IN_LDS)
+            {
+#pragma unroll
+                for (int q = 0; q < NKEEP; ++q)
+                    keep[q] = sm[L::oBE + (q * NT + tid < KEEP ? q * NT + tid : 0)];
+                kept = IN_REG;
+            }
+            else if (again && kept == IN_REG)
+            {
+#pragma unroll
+                for (int q = 0; q < NKEEP; ++q)
+                    if (q * NT + tid < KEEP) sm[L::oBE + q * NT + tid] = keep[q];
+                psync<WAVE>();
+            }
+            if (i == 1) kept = IN_LDS;
             // an opaque lane index (range restored): the lane's addresses are formed in each iteration,
             // not kept from the kernel's entry and spilled (net86 Helmholtz FP64: 67 -> 19 VGPRs, net14
             // 137 -> 84; 524,288 net86 particles 568 -> 536 ms, 4,099 of net87 at cap 2,000 95 -> 87 ms)
@@ -1696,7 +1716,7 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
                 elapsed += timestep;
                 ++n_sub;
                 cyc.lim = 0;
-                kept    = false;
+                kept    = NONE;
                 if ((dt_tot - elapsed) / dt_tot < k::substep_dtTol) break;
             }
             else if (i == 0)
