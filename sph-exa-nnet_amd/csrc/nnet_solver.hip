@@ -501,15 +501,13 @@ struct TileLU
             asm volatile("" : "+v"(lane));
             lane &= 63;
         }
-        // the U entries of four columns are loaded ahead of their four dependent steps (a
-        // scheduling barrier keeps each group's loads together), so the v_readlane/FMA chain does
-        // not wait for LDS at every step (groups of 4 measured faster than 8 and 16: fewer live
-        // registers)
+        // the U entries of four columns are loaded one group ahead of their four dependent steps, so
+        // the v_readlane/FMA chain does not wait for LDS (scheduling barriers keep each group's loads
+        // together).  net86, one retried iteration with this and the fill below: 20.8 -> 20.3 us.
         constexpr int NA = (N + 63) / 64, G = 4;
-#pragma unroll
-        for (int j0 = N - 1; j0 > 0; j0 -= G)
+        R             u[2][G][NA];
+        auto load = [&](R (&b)[G][NA], int j0) __attribute__((always_inline))
         {
-            R u[G][NA];
 #pragma unroll
             for (int s = 0; s < G; ++s)
 #pragma unroll
@@ -521,8 +519,14 @@ struct TileLU
                     // diagonal, j <= 0)
                     const bool ok = j > 0 && row < j;
                     const R    x  = sU[ok ? uidx(row, j) : 0];
-                    u[s][a]       = ok ? x : R(0);
+                    b[s][a]       = ok ? x : R(0);
                 }
+        };
+        load(u[0], N - 1);
+#pragma unroll
+        for (int j0 = N - 1, g = 0; j0 > 0; j0 -= G, ++g)
+        {
+            if (j0 > G) load(u[(g + 1) & 1], j0 - G);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int s = 0; s < G; ++s)
@@ -535,7 +539,7 @@ struct TileLU
                     for (int a = 0; a <= (j - 1) >> 6; ++a)
                     {
                         const int row = lane + 64 * a;
-                        if (row < j) acc[a] = fma(-u[s][a], xj, acc[a]);
+                        if (row < j) acc[a] = fma(-u[g & 1][s][a], xj, acc[a]);
                     }
                 }
             }
@@ -1451,16 +1455,15 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
             };
             // the lane's register slots (tile placement of TileLU) filled from the Jacobian
             // non-zeros, which are numbered lane-major in slot order
-            // Every slot first takes its Jacobian-block value (rows and columns 1 .. N-1, zero
-            // elsewhere) without branches; then the few slots of column 0 (dY/dT), column N (the
+            // Every slot first takes its Jacobian-block value (zero outside the pattern) without
+            // branches; then the few slots of column 0 (dY/dT), column N (the
             // right-hand side) and row 0 (temperature) are overwritten where they sit: column 0 in
             // register lane column 0 of tile column 0, column N in lane column N & 15 of tile column
             // N >> 4, row 0 in register 0 of lane row 0 of tile row 0.  Each slot gets the value
             // entry() gives it.
             auto fill = [&](auto& Mt) __attribute__((always_inline))
             {
-                const uint64_t mask = (uint64_t)lmap.x | ((uint64_t)lmap.y << 32);
-                const int      base = (int)lmap.z; // id of this lane's first non-zero
+                int nzi = (int)lmap.z; // this lane's next non-zero: they are numbered in slot order
 #pragma unroll
                 for (int ti = 0; ti < TI; ++ti)
 #pragma unroll
@@ -1468,15 +1471,18 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
 #pragma unroll
                         for (int v = 0; v < 4; ++v)
                         {
-                            const int  slot = (ti * TI + tj) * 4 + v;
-                            const int  ri = tile_row(wr + WR * ti, lr, v), ci = tile_col(wc + WR * tj, lc);
-                            const bool nz = (mask >> slot) & 1;
-                            // the lane's non-zeros are numbered in slot order
-                            const int    nzi = base + (int)__popcll(mask & ((1ull << slot) - 1ull));
-                            const double Jl  = sJv[nz ? nzi : 0];
-                            const double J   = nz ? Jl : 0.;
-                            const double x   = (ci == ri) ? 1. - thdt * J : mthdt * J;
-                            Mt[ti][tj][v]    = (ri >= 1 && ri < N && ci >= 1 && ci < N) ? x : 0.;
+                            const int    slot = (ti * TI + tj) * 4 + v;
+                            const int    nz   = ((slot < 32 ? lmap.x : lmap.y) >> (slot & 31)) & 1;
+                            const double Jl   = sJv[nz ? nzi : 0];
+                            nzi += nz;
+                            // -thdt J, on the diagonal 1 - thdt J (mthdt is -thdt)
+                            double x = mthdt * (nz ? Jl : 0.);
+                            if (ti == tj)
+                            {
+                                const int ri = tile_row(wr + WR * ti, lr, v), ci = tile_col(wc + WR * tj, lc);
+                                if (ci == ri && ri < N) x = 1. + x;
+                            }
+                            Mt[ti][tj][v] = x;
                         }
                 // column 0: dY/dT
                 if (wc == 0 && lc == 0)
