@@ -83,7 +83,8 @@ struct Lds
     // the LU they hold the refinement residual.  Eight-pivot LU: two generations of panel columns
     // [row][PANEL8] (its pivot rows go straight into the packed rows).
     static constexpr int oPan = ((oRow0 + (MIX ? N + 1 : 0)) + 3) & ~3, panWords = (LU8 ? 2 * PANEL8 : 16) * NPAD,
-                         oCyc = oPan + panWords, total = oCyc + 3 * (C::NT / 64); // a Cycle per wavefront
+                         oCyc = oPan + panWords,
+                         total = (oCyc + 3 * (C::NT / 64) + 1) & ~1; // a Cycle per wavefront
 };
 
 // Exact cycles of rejected attempts.  A rejected attempt restarts from the same accepted state, so

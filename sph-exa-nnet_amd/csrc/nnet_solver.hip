@@ -8,9 +8,10 @@
 //              values the reference's scatter loops, nuclear_net.hpp:347-438, produce), then the
 //              (d+1)x(d+2) augmented Newton matrix is filled directly into registers as 16x16
 //              tiles in the v_mfma_f64_16x16x4f64 result layout.
-//   LU         right-looking unpivoted elimination on the register-resident tiles, blocks of
-//              four pivots, rank-4 trailing updates on MFMA (eigen.hpp:179-206); the normalised
-//              pivot rows are staged in LDS, which also serves the back substitution.
+//   LU         right-looking unpivoted elimination (eigen.hpp:179-206).  net86 / net87: on the
+//              register-resident tiles, FP64 in blocks of eight pivots, FP32 (mixed precision) of
+//              four, trailing updates on MFMA; the normalised pivot rows are staged in LDS, which
+//              also serves the back substitution.  net14 FP64: one row per lane.
 //   controller the substep/Newton state machine of nuclear_net.hpp:692-959 is replicated in
 //              every lane (uniform control flow) with exact replay-stall detection.
 // Persistent workgroups (as many as are resident at once) take particles from a device work queue,
@@ -175,7 +176,8 @@ __device__ __forceinline__ double pow_count(double x, int n)
 __device__ __forceinline__ double factorial_count(int n) { return n == 2 ? 2. : n == 3 ? 6. : n == 4 ? 24. : 1.; }
 
 // ---------------------------------------------------------------------------------------------
-// Tile LU.  The augmented (N x N+1) Newton matrix lives in registers as 16x16 FP64 tiles in the
+// Tile LU (the mixed path's FP32 factorization; its triangular solves serve FP64 too).  The
+// augmented (N x N+1) Newton matrix lives in registers as 16x16 tiles in the
 // result layout of v_mfma_f64_16x16x4f64: register v of lane l of a tile holds row 16*I + (l>>4)
 // + 4v, column 16*J + (l&15).  Wave (wr, wc) of the WR x WR wave grid owns tiles (wr + WR*ti,
 // wc + WR*tj).  Elimination proceeds in blocks of four pivots (eigen.hpp:182-206 order per
@@ -836,6 +838,85 @@ struct PanelLU
         publish<0>(Mt, pan, sU, w / WR, w % WR, lane >> 4, lane & 15);
         __syncthreads();
         step<0>(Mt, pan, sU, w, lane);
+    }
+};
+
+// value of x in lane row G (lanes 16 G .. 16 G + 15), lane by lane, in all four lane rows
+template<int G>
+__device__ __forceinline__ unsigned lane_row(unsigned x)
+{
+    const auto     p = __builtin_amdgcn_permlane16_swap(x, x, false, false); // rows {0,0,2,2}, {1,1,3,3}
+    const unsigned v = p[G & 1];
+    const auto     q = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return q[G >> 1];
+}
+template<int G>
+__device__ __forceinline__ double lane_row(double x)
+{
+    const unsigned long long b  = __double_as_longlong(x);
+    const unsigned           lo = lane_row<G>((unsigned)b), hi = lane_row<G>((unsigned)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// ---------------------------------------------------------------------------------------------
+// LU and back substitution of the FP64 net14 solve (15 x 16 augmented, one wavefront) with the
+// arithmetic per element of the tile LU.  The system is too small to be bound by anything but the
+// chain of its 15 pivots, and blocks of four spent it on LDS round trips (panel, multipliers,
+// normalised rows) and 4x4 factors.  Here one row sits in each lane of a 16-lane row, four of its
+// columns in each of the four lane rows: a pivot's row reaches the others through DPP row
+// broadcasts, its column through lane-row swaps beside the reciprocal, and LDS is passed once, from
+// the tile layout of the fill.  One retried net14 iteration 4.86 -> 3.84 us, a full one 17.9 ->
+// 17.3; 50,021 particles, first step, 83.7 -> 73.0 ms.
+// ---------------------------------------------------------------------------------------------
+struct RowLU
+{
+    static constexpr int N = Cfg<14>::N, STRIDE = 18; // LDS row stride (doubles, 16-byte aligned rows)
+    static_assert(N == 15 && 16 * STRIDE <= Lds<14, false>::headEnd, "16 x 16 entries in the dead head arrays");
+    static_assert(Lds<14, false>::total % 2 == 0, "16-byte aligned particle groups");
+
+    static __device__ __forceinline__ void solve(const dx4& Mt, double* sM, double* sX, int lane)
+    {
+        const int lr = lane >> 4, lc = lane & 15;
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            sM[tile_row(0, lr, v) * STRIDE + lc] = Mt[v];
+        psync<true>();
+        // row lc, columns 4 lr .. 4 lr + 3
+        const double2* r = reinterpret_cast<const double2*>(sM + lc * STRIDE + 4 * lr);
+        double         a[4] = {r[0].x, r[0].y, r[1].x, r[1].y};
+        double         rl = 0.; // reciprocal of the row's pivot
+        static_for<N>(
+            [&](auto pc) __attribute__((always_inline))
+            {
+                constexpr int p = decltype(pc)::value, g = p >> 2, c = p & 3;
+                const double  rinv = TileT<double>::recip(bcast_lane(a[c], 16 * g + p));
+                // multipliers of the rows below (|w| <= 1e-40 counts as zero); the others' are zero
+                const double col = lane_row<g>(a[c]);
+                const bool   ok  = (lc > p) & (fabs(col) > k::epsilonSystem);
+                const double w   = ok ? col : 0.;
+                rl               = lc == p ? rinv : rl;
+                // columns left of the pivot take part with whatever they hold: nothing reads them again
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    a[j] = fma(-w, row_bcast<p>(a[j] * rinv), a[j]);
+            });
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            a[j] *= rl;
+        // back substitution, columns descending: x_j is subtracted from every row above it in the lane
+        // row that holds column j (the other lane rows run along; the sums move with the columns)
+        double acc = lane_row<3>(a[3]);
+        static_for<N - 1>(
+            [&](auto jc) __attribute__((always_inline))
+            {
+                constexpr int j = N - 1 - decltype(jc)::value, g = j >> 2;
+                const double  xj = bcast_lane(acc, 16 * g + j);
+                const double  y  = fma(-a[j & 3], xj, acc);
+                acc              = lc < j ? y : acc;
+                if constexpr ((j & 3) == 0) acc = lane_row<g>(acc);
+            });
+        if (lane < N) sX[lane] = acc;
+        psync<true>();
     }
 };
 
@@ -1523,15 +1604,14 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
             {
                 dx4 Mt[TI][TI];
                 fill(Mt);
-                // the packed rows the LU writes alias the arrays the fill reads: the barrier after
-                // the LU's first panel publish (which writes only the panel buffers) orders every
-                // lane's fill before the first packed-row store
-                // ---- LU (eigen.hpp:179-206), four pivots per block ----
-                if constexpr (L::LU8)
-                    PanelLU<NET>::factor(Mt, sPan, sU, __builtin_amdgcn_readfirstlane(tid >> 6), tid & 63);
+                // ---- LU (eigen.hpp:179-206) and back substitution (eigen.hpp:208-221) ----
+                if constexpr (NET == 14)
+                {
+                    RowLU::solve(Mt[0][0], sm, sX, tid);
+                    return;
+                }
                 else
-                    TileLU<NET, double, false, WAVE>::factor(Mt, sPan, sU, nullptr, nullptr, wr, wc, lr, lc, tid);
-                // ---- back substitution (eigen.hpp:208-221) ----
+                    PanelLU<NET>::factor(Mt, sPan, sU, __builtin_amdgcn_readfirstlane(tid >> 6), tid & 63);
                 if (tid < 64)
                 {
                     double acc[NA];
