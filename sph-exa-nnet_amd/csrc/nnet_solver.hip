@@ -1586,21 +1586,27 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
                             const int ri = tile_row(wr + WR * ti, lr, v);
                             if (ri >= 1 && ri < N) Mt[ti][JN / WR][v] = entry(ri, N, 0.);
                         }
-                // row 0 (temperature)
+                // row 0 (temperature): entry()'s three forms with one quotient
                 if (wr == 0 && lr == 0)
 #pragma unroll
                     for (int tj = 0; tj < TI; ++tj)
                     {
-                        const int ci = tile_col(wc + WR * tj, lc);
+                        const int    ci = tile_col(wc + WR * tj, lc);
+                        const double be = sBE[ci < 1 ? 0 : ci < N ? ci - 1 : D - 1];
+                        const double q  = (ci == 0 ? k::theta * value_1 : ci < N ? -be : T * value_1) / cvv;
+                        const double x  = ci == 0 ? 1 - q : q;
                         if (ci <= N)
                         {
-                            const double x = entry(0, ci, 0.);
-                            Mt[0][tj][0]   = x;
+                            Mt[0][tj][0] = x;
                             if constexpr (MIX) sRow0[ci] = x;
                         }
                     }
             };
-            auto solve_fp64 = [&]() __attribute__((always_inline))
+            // the FP64 solve of net86 / net87 leaves the NaN test of the new abundances in s_flag: the
+            // wavefront that solves has them all, and the controller's own vote would cost the
+            // workgroup a reduction
+            constexpr bool SOLVER_NAN = NET != 14 && !MIX;
+            auto           solve_fp64 = [&]() __attribute__((always_inline))
             {
                 dx4 Mt[TI][TI];
                 fill(Mt);
@@ -1623,9 +1629,20 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
                         acc[a]         = row < N ? x : 0.;
                     }
                     TileLU<NET, double, false, WAVE>::back(sU, acc, tid);
+                    // (and whether an abundance becomes NaN, for the controller)
+                    bool bad = false;
 #pragma unroll
                     for (int a = 0; a < NA; ++a)
-                        if (tid + 64 * a < N) sX[tid + 64 * a] = acc[a];
+                    {
+                        const int row = tid + 64 * a;
+                        if (row < N) sX[row] = acc[a];
+                        if (row >= 1 && row < N) bad = bad || isnan(sY[row - 1] + acc[a]);
+                    }
+                    if constexpr (SOLVER_NAN)
+                    {
+                        const bool any = __any(bad);
+                        if (tid == 0) s_flag = any ? 1u : 0u;
+                    }
                 }
                 psync<WAVE>();
             };
@@ -1754,7 +1771,7 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
                 yb_new  = sY[tid] + sX[tid + 1];
                 nanflag = isnan(yb_new) ? 1 : 0;
             }
-            const bool has_nan = psync_or<WAVE>(nanflag) || isnan(T_new);
+            const bool has_nan = (SOLVER_NAN ? s_flag != 0 : psync_or<NT == 64>(nanflag)) || isnan(T_new);
             if (has_nan || T_new < 0)
             {
                 u *= k::nanDtStep;
