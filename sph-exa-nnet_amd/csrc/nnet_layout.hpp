@@ -60,7 +60,8 @@ struct Lds
     static constexpr int D = C::D, N = C::N, NR = C::NR, NE = C::NE;
     static constexpr int NU = N * (N + 1) / 2; // packed normalised rows (columns k+1 .. N)
     static constexpr int NL = N * (N - 1) / 2; // packed multipliers (columns 0 .. k-1)
-    // head: rate and mass-action arrays, dead once the Jacobian is summed
+    // head: rate and mass-action arrays, dead once the Jacobian is summed (the NR words at oJok are
+    // spare: a reaction without derivative holds zeros at oTr)
     static constexpr int oMu = 0, oEff = oMu + D, oDeff = oEff + NE, oL = oDeff + NE, oDl = oL + NE,
                          oRate = oDl + NE, oDrate = oRate + NR, oVal = oDrate + NR, oDval = oVal + NR,
                          oTr = oDval + NR, oJok = oTr + NR * MAXQ, headEnd = oJok + NR;
