@@ -127,6 +127,16 @@ def helm_table_read(path):
     return out
 
 
+def _row_pointers(Y):
+    """Device addresses of the rows of a (d x n) tensor, or of a list of d tensors.  A tensor's rows
+    are stepped through by its stride: indexing would make a tensor of each row (14 of them took
+    more host time than the launch of an EOS refresh)."""
+    if not hasattr(Y, "stride") or Y.dim() < 2 or Y.numel() == 0:
+        return [Y[s].data_ptr() for s in range(len(Y))]
+    base, step = Y.data_ptr(), Y.stride(0) * Y.element_size()
+    return [base + s * step for s in range(Y.shape[0])]
+
+
 class Context:
     """One HIP device context (tables uploaded once)."""
 
@@ -247,10 +257,10 @@ class Context:
         """Post-step EOS refresh (computeHelmEOS): Y is a (dim x n) device tensor (or a list of dim
         per-species device tensors), temp and rho device tensors of n doubles, `out` a dict whose
         keys among u, cv, p, c, dpdT name the device tensors to fill (others are skipped)."""
-        rows = [Y[s] for s in range(len(Y))]
+        rows = _row_pointers(Y)
         n = temp.shape[0]
         zarr = (C.c_double * len(Z))(*[float(z) for z in Z])
-        yp = (C.c_void_p * len(rows))(*[r.data_ptr() for r in rows])
+        yp = (C.c_void_p * len(rows))(*rows)
         o = [out[k].data_ptr() if out.get(k) is not None else None for k in ("u", "cv", "p", "c", "dpdT")]
         args = [self.h, n, len(rows), zarr, temp.data_ptr(), rho.data_ptr(), yp] + o
         if sync and stream is None:
