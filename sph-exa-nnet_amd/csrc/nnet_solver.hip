@@ -940,13 +940,14 @@ __device__ __forceinline__ void in_groups(int& e, int e1, F&& f)
 // queue and integrate each over one hydro step, until the queue is empty.  sm: the group's
 // Lds<NET, MIX>::total doubles of LDS; simg: the network's assembly image, staged in LDS by the
 // caller; s_pf: two LDS words of the group; tid: the lane's index in the group.  WAVE: the group
-// is one wavefront that shares its workgroup with other groups (wavefront barriers only).
+// is one wavefront that shares its workgroup with other groups (wavefront barriers only); groups:
+// particle groups per workgroup.
 // EosT / BatchT: the EOS and batch descriptions (EosDev / BatchDev, or views of the same fields).
 // ---------------------------------------------------------------------------------------------
 template<int NET, int EOSK, bool MIX, bool WAVE, class EosT, class BatchT>
 __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed, const BatchT& bd,
                                                 const StepParams& sp, double* sm, const uint32_t* simg,
-                                                unsigned* s_pf, int tid)
+                                                unsigned* s_pf, int tid, unsigned groups)
 {
     using C  = Cfg<NET>;
     using L  = Lds<NET, MIX>;
@@ -1003,7 +1004,7 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
     // the particles) and for 83% on net14's (60%).  Not where every particle starts at once.
     // 524,288 net86 particles, first step: 364 -> 280 ms; 50,021 of net14 68.5 -> 65.8.
     const unsigned nq    = (unsigned)(q1 - q0), // at most 2^31 particles fit a GPU
-                   times = !bd.order && nq > gridDim.x * (blockDim.x / NT) ? 2 : 1;
+                   times = !bd.order && nq > gridDim.x * groups ? 2 : 1;
     for (;;)
     {
         psync<WAVE>();
@@ -1222,11 +1223,14 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
                         reverse(exp(el));
                     }
                     // species lanes: net14 the first lanes, net86 / net87 those after the fitted rates'
-                    const int s = NET == 14 ? k : tid - nd.nfit;
+                    // (the radius is broadcast outside the branch: inside it the lane that holds it may
+                    // be inactive, and a register copied or reloaded there keeps the active lanes only)
+                    const int    s  = NET == 14 ? k : tid - nd.nfit;
+                    const double ae = bcast_lane(pv, spx::PAE);
                     if (s >= 0 && s < Dr)
                     {
                         double be, mu;
-                        species_coulomb(Tg, bcast_lane(pv, spx::PAE), nd.Z53[s], nd.BE0[s], be, mu);
+                        species_coulomb(Tg, ae, nd.Z53[s], nd.BE0[s], be, mu);
                         if (NET != 14 && s == 1) mu = 0; // neutron (net86.cpp:603)
                         sBE[s] = be;
                         sMu[s] = mu;
@@ -1892,7 +1896,8 @@ __global__ void __launch_bounds__(Cfg<NET>::NT * PPW, Cfg<NET>::WPE)
     for (int w = threadIdx.x; w < nd.img_words; w += C::NT * PPW)
         simg[w] = nd.img[w];
     __syncthreads();
-    solve_particles<NET, EOSK, MIX, (PPW > 1)>(nd, ed, bd, sp, sm + group * L::total, simg, s_pf + 2 * group, tid);
+    solve_particles<NET, EOSK, MIX, (PPW > 1)>(nd, ed, bd, sp, sm + group * L::total, simg, s_pf + 2 * group, tid,
+                                                 PPW);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1962,19 +1967,19 @@ __global__ void __launch_bounds__(FUSE_NT, 2) nnet_solve_fused(FusedDev fd, Step
         if (P.kind == 87)
         {
             asm volatile("" : "+v"(t));
-            solve_particles<87, EOSK, MIX, false>(nd, ev, bv, sp, sm, simg, s_pf, t);
+            solve_particles<87, EOSK, MIX, false>(nd, ev, bv, sp, sm, simg, s_pf, t, 1);
         }
         else if (P.kind == 86)
         {
             asm volatile("" : "+v"(t));
-            solve_particles<86, EOSK, MIX, false>(nd, ev, bv, sp, sm, simg, s_pf, t);
+            solve_particles<86, EOSK, MIX, false>(nd, ev, bv, sp, sm, simg, s_pf, t, 1);
         }
         else
         {
             asm volatile("" : "+v"(t));
             const int g = t >> 6;
             solve_particles<14, EOSK, MIX, true>(nd, ev, bv, sp, sm + g * Lds<14, MIX>::total, simg, s_pf + 2 * g,
-                                                 t & 63);
+                                                 t & 63, FUSE_NT / 64);
         }
     }
 }
