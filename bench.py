@@ -465,6 +465,9 @@ def main():
                      "traffic_source": "constant: calibrated rocprofv3 FETCH_SIZE/WRITE_SIZE of the profile run",
                      "kernel": f"nnet_solve_kernel<{cfg['net']}, HELMHOLTZ, FP64>",
                      # the kernel is latency x slot bound: iterations/s = slots / iteration latency
+                     # the device's counts are those of running every attempt: whole periods of exact
+                     # cycles are counted, not run
+                     "achieved_from": "counted Newton iterations (exact cycles included)",
                      "limiter": "latency",
                      "latency_model": {"resident_slots": slots, "iteration_latency_us": dom["iteration_latency_us"],
                                        "newton_iters_per_s": dom["newton_iters_per_s"]}},
