@@ -106,7 +106,8 @@ typedef struct nnet_batch {
     const double* Z;      /* HelmholtzFunctor(Z, z_dim): host array of z_dim charges */
     int z_dim;
     int precision;        /* NNET_PRECISION_* */
-    size_t n;             /* particles [0, n) of the arrays below */
+    size_t n;             /* particles [0, n) of the arrays below; at most 2^32 - 1 minus 32 for
+                             each compute unit of the device */
     const double* rho;    /* device, n */
     double* rho_m1;       /* device, n (read/written only if use_drhodt) */
     double* const* Y;     /* host array of n_species device pointers, each n molar abundances */

@@ -126,6 +126,17 @@ __attribute__((always_inline)) constexpr long cycle_skip(Cycle& c, uint64_t dt, 
     return 0;
 }
 
+// The work queue of a launch is a 32-bit count of the positions taken so far; every particle group
+// takes one past the end before it stops.  How often the queue runs over its nq particles in a launch
+// of `groups` particle groups: twice (dense particles first, solve_particles) without an order and with
+// more particles than start at once, but only where twice the count still fits.
+__attribute__((always_inline)) constexpr uint32_t queue_passes(uint32_t nq, uint32_t groups, bool ordered)
+{
+    return !ordered && nq > groups && nq <= (0xffffffffu - groups) / 2 ? 2 : 1;
+}
+// Particles of one launch at most, on a device of n_cu compute units (32 wavefronts each).
+constexpr uint64_t queue_limit(uint32_t n_cu) { return 0xffffffffull - 32ull * n_cu; }
+
 // Jacobian non-zero slot (position in the image's descending-length order) that lane `tid` of a
 // particle's NT lanes sums in pass `pass`, or a value >= nnz when it has none: pass p takes slot
 // tid + NT p; with four wavefronts the slots beyond three full passes go to wavefront 1 (no species

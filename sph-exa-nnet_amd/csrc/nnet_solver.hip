@@ -1003,8 +1003,8 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
     // rho >= 1e7 g/cm^3 holds for all of them on the net86 and net87 Helmholtz sets (30% and all of
     // the particles) and for 83% on net14's (60%).  Not where every particle starts at once.
     // 524,288 net86 particles, first step: 364 -> 280 ms; 50,021 of net14 68.5 -> 65.8.
-    const unsigned nq    = (unsigned)(q1 - q0), // at most 2^31 particles fit a GPU
-                   times = !bd.order && nq > gridDim.x * groups ? 2 : 1;
+    const unsigned nq    = (unsigned)(q1 - q0), // (the host refuses more than queue_limit)
+                   times = queue_passes(nq, gridDim.x * groups, bd.order != nullptr);
     for (;;)
     {
         psync<WAVE>();
@@ -2473,6 +2473,8 @@ static int check_call(nnet_ctx* c, const nnet_batch* batches, int nb, double hyd
         if (!b.network || b.network->ctx != c) return fail(c, NNET_E_ARG, "batch without a network of this context");
         if (b.n == 0) continue;
         ++n_live;
+        if (b.n > queue_limit((uint32_t)c->n_cu))
+            return fail(c, NNET_E_ARG, "at most " + std::to_string(queue_limit((uint32_t)c->n_cu)) + " particles per batch");
         if (!b.rho || !b.Y || !b.temp || !b.dt || (use_drhodt != NNET_DRHODT_OFF && !b.rho_m1))
             return fail(c, NNET_E_ARG, "null particle array");
         if (b.precision != NNET_PRECISION_FP64 && b.precision != NNET_PRECISION_MIXED)
