@@ -123,6 +123,9 @@ struct EosView : EosCore
     const double* Z;
 };
 
+// Word of a batch's counters that says whether a launch without an order takes dense particles first
+// (in calls with a routing hint, which have an order, it is the queue of the routed pass).
+constexpr int QPLAN = 1;
 struct BatchCore
 {
     size_t        n;
@@ -1001,10 +1004,11 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
     // others to the second time.  A particle that runs into the iteration cap takes as long as the
     // rest of the call, and the call as long as both when it is met late.  Such particles are dense:
     // rho >= 1e7 g/cm^3 holds for all of them on the net86 and net87 Helmholtz sets (30% and all of
-    // the particles) and for 83% on net14's (60%).  Not where every particle starts at once.
+    // the particles) and for 83% on net14's (60%).  Not where every particle starts at once, nor where
+    // much of the batch does not burn (nnet_queue_plan).
     // 524,288 net86 particles, first step: 364 -> 280 ms; 50,021 of net14 68.5 -> 65.8.
     const unsigned nq    = (unsigned)(q1 - q0), // (the host refuses more than queue_limit)
-                   times = queue_passes(nq, gridDim.x * groups, bd.order != nullptr);
+                   times = queue_passes(nq, gridDim.x * groups, bd.order || bd.queue[QPLAN] == 0u);
     for (;;)
     {
         psync<WAVE>();
@@ -2086,6 +2090,19 @@ __global__ void nnet_queue_reset(unsigned int* q, int n)
     if (i < n) q[i] = 0u;
 }
 
+// The reset of a batch's counters in a call without an order and with more particles than start at
+// once: also decides, from particles spread over the batch, whether dense particles go first
+// (dense_first_pays; one pair of loads per lane, so it takes a plain reset's time and their latency).
+__global__ void __launch_bounds__(PLAN_SAMPLE)
+    nnet_queue_plan(unsigned int* q, int nctr, const double* __restrict__ rho, const double* __restrict__ temp, size_t n)
+{
+    const int    i    = threadIdx.x;
+    const size_t p    = (size_t)((unsigned long long)n * i / PLAN_SAMPLE);
+    const bool   idle = !(rho[p] > k::minRho && temp[p] > k::minTemp);
+    const int    cnt  = __syncthreads_count(idle);
+    if (i < nctr) q[i] = i == QPLAN && dense_first_pays((unsigned)cnt) ? 1u : 0u;
+}
+
 // ---------------------------------------------------------------------------------------------
 // Cost-ordered dispatch: particles are handed to the persistent workgroups in descending buckets
 // of an expected cost (the caller's hint, e.g. the Newton iterations of the previous call), so the
@@ -2196,7 +2213,8 @@ struct nnet_ctx
     double*   d_cells3 = nullptr;
     bool      helm_ok  = false;
     // NCTR counters per batch of a call: work queues of the first pass, of the routed FP64 pass
-    // and of the redo pass; then the redo range {0, count}
+    // (without an order: the plan of the first, QPLAN) and of the redo pass; then the redo range
+    // {0, count}
     static constexpr int NCTR = 5;
     unsigned int* d_queue = nullptr;
     int           n_queue = 0; // batches the counters cover
@@ -2540,6 +2558,17 @@ static const uint32_t* enqueue_order(const nnet_batch& b, int bi, const uint32_t
     return order;
 }
 
+// Zeroes a batch's counters; plan: decide there whether dense particles go first, too (a launch without
+// an order and with more particles than start at once)
+static void reset_queue(const nnet_batch& b, unsigned int* ctr, bool plan, hipStream_t s)
+{
+    if (plan)
+        hipLaunchKernelGGL(nnet_queue_plan, dim3(1), dim3(PLAN_SAMPLE), 0, s, ctr, nnet_ctx::NCTR, b.rho,
+                           (const double*)b.temp, b.n);
+    else
+        hipLaunchKernelGGL(nnet_queue_reset, dim3(1), dim3(64), 0, s, ctr, nnet_ctx::NCTR);
+}
+
 // Can the call's batches run as one fused launch?  All live batches share the EOS and the
 // precision, there are at most FUSE_PHASES of them, and their abundance pointers and charges fit
 // the FUSE_SPECIES-entry arrays of the launch arguments.
@@ -2579,6 +2608,20 @@ static int enqueue_fused(nnet_ctx* c, const nnet_batch* batches, int nb, double 
     FusedDev   fd{}, fr{};
     size_t     order_off = 0, redo_off = 0, work = 0;
     int        zoff = 0, yoff = 0;
+    for (int bi : phase)
+        work += batches[bi].network->kind == 14 ? (batches[bi].n + 3) / 4 : batches[bi].n;
+    // workgroups of a launch: as many as are resident at once, at most one per particle (net14: four)
+    auto wgs_of = [&](auto kern)
+    {
+        int per_cu = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, FUSE_NT, 0) != hipSuccess || per_cu < 1)
+            per_cu = 1;
+        return std::min<size_t>(work, (size_t)per_cu * c->n_cu);
+    };
+    const size_t wgs = eos == NNET_EOS_IDEAL ? (mix ? wgs_of(nnet_solve_fused<NNET_EOS_IDEAL, true>)
+                                                    : wgs_of(nnet_solve_fused<NNET_EOS_IDEAL, false>))
+                                             : (mix ? wgs_of(nnet_solve_fused<NNET_EOS_HELMHOLTZ, true>)
+                                                    : wgs_of(nnet_solve_fused<NNET_EOS_HELMHOLTZ, false>));
     fd.nphase = fr.nphase = (int)phase.size();
     for (int k = 0; k < (int)phase.size(); ++k)
     {
@@ -2586,7 +2629,6 @@ static int enqueue_fused(nnet_ctx* c, const nnet_batch* batches, int nb, double 
         const nnet_batch& b   = batches[bi];
         const int         d   = b.network->d;
         unsigned int*     ctr = bufs.queue + (size_t)nnet_ctx::NCTR * bi;
-        hipLaunchKernelGGL(nnet_queue_reset, dim3(1), dim3(64), 0, st, ctr, nnet_ctx::NCTR);
         PhaseDev& P = fd.ph[k];
         P.nd        = b.network->d_dev;
         P.kind      = b.network->kind;
@@ -2618,23 +2660,19 @@ static int enqueue_fused(nnet_ctx* c, const nnet_batch* batches, int nb, double 
         }
         const unsigned int* range = nullptr;
         bc.order                  = enqueue_order(b, bi, nullptr, bufs, order_off, st, range);
+        reset_queue(b, ctr, !bc.order && b.n > wgs * (P.kind == 14 ? FUSE_NT / 64 : 1), st);
         // the FP64 pass over the redo list: its own queue, the list as the order, {0, count}
         fr.ph[k]             = P;
         fr.ph[k].b.queue     = ctr + 2;
         fr.ph[k].b.order     = bc.redo;
         fr.ph[k].b.qrange    = ctr + 3;
         fr.ph[k].b.fp64_pass = 1;
-        work += P.kind == 14 ? (b.n + 3) / 4 : b.n;
     }
     std::memcpy(fr.Z, fd.Z, sizeof(fd.Z));
     std::memcpy(fr.Y, fd.Y, sizeof(fd.Y));
     auto go = [&](auto kern, const FusedDev& a, const StepParams& s)
     {
-        int per_cu = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, FUSE_NT, 0) != hipSuccess || per_cu < 1)
-            per_cu = 1;
-        const size_t wgs = std::min<size_t>(work, (size_t)per_cu * c->n_cu);
-        hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(FUSE_NT), 0, st, a, s);
+        hipLaunchKernelGGL(kern, dim3((unsigned)wgs_of(kern)), dim3(FUSE_NT), 0, st, a, s);
     };
     if (eos == NNET_EOS_IDEAL)
     {
@@ -2704,7 +2742,6 @@ static int enqueue_compute(nnet_ctx* c, const nnet_batch* batches, int nb, doubl
         const NetDev& nd  = b.network->dev;
         unsigned int* ctr = bufs.queue + (size_t)nnet_ctx::NCTR * bi;
         bd.queue          = ctr;
-        hipLaunchKernelGGL(nnet_queue_reset, dim3(1), dim3(64), 0, bst, ctr, nnet_ctx::NCTR);
         const bool mix = b.precision == NNET_PRECISION_MIXED;
         if (mix)
         {
@@ -2715,6 +2752,8 @@ static int enqueue_compute(nnet_ctx* c, const nnet_batch* batches, int nb, doubl
         const uint32_t*     route = (mix && allow_route) ? b.fp64_hint : nullptr;
         const unsigned int* range = nullptr;
         bd.order                  = enqueue_order(b, bi, route, bufs, order_off, bst, range);
+        bool reset = bd.order != nullptr; // without an order: with the first launch, which knows its groups
+        if (reset) reset_queue(b, ctr, false, bst);
         const int         kind = b.network->kind;
         const int         ak   = fork ? (live - 1) % nnet_ctx::NSIDE : 0;
         const hipStream_t ast  = c->aux[ak];
@@ -2737,6 +2776,8 @@ static int enqueue_compute(nnet_ctx* c, const nnet_batch* batches, int nb, doubl
                 if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, nt, 0) != hipSuccess || per_cu < 1)
                     per_cu = 1;
                 const size_t wgs = std::min<size_t>((b.n + ppw - 1) / ppw, (size_t)per_cu * c->n_cu);
+                if (!reset) reset_queue(b, ctr, b.n > wgs * ppw, s);
+                reset = true;
                 hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(nt), 0, s, nd, ed, bdv, spv);
             };
             const int ppw = c->tuning.ppw(NV, EV, MV);
