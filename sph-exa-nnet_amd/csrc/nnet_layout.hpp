@@ -146,6 +146,19 @@ constexpr bool     dense_first_pays(uint32_t idle) { return 4 * idle <= PLAN_SAM
 // Particles of one launch at most, on a device of n_cu compute units (32 wavefronts each).
 constexpr uint64_t queue_limit(uint32_t n_cu) { return 0xffffffffull - 32ull * n_cu; }
 
+// Place of a particle in an ordered call, highest first: the bit length of its count (an earlier
+// step's Newton iterations).  A dense particle that burns and has no count yet (a first step) goes
+// first, as in a call without an order: 60,013 net86 particles, two steps at cap 2,000: 91.2 -> 86.2 ms.
+// A cold one's count stays 0 in every step; it goes last, not in front of the long ones (four long net14
+// particles among 1,000,000 cold dense ones: 18.8 -> 17.4 ms).
+constexpr int NBUCKET = 32;
+__attribute__((always_inline)) constexpr int order_bucket(uint32_t count, bool dense_burning)
+{
+    if (count == 0) return dense_burning ? NBUCKET - 1 : 0;
+    const int b = 32 - __builtin_clz(count);
+    return b < NBUCKET ? b : NBUCKET - 1;
+}
+
 // Jacobian non-zero slot (position in the image's descending-length order) that lane `tid` of a
 // particle's NT lanes sums in pass `pass`, or a value >= nnz when it has none: pass p takes slot
 // tid + NT p; with four wavefronts the slots beyond three full passes go to wavefront 1 (no species

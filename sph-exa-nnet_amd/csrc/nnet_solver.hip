@@ -2108,36 +2108,29 @@ __global__ void __launch_bounds__(PLAN_SAMPLE)
 // of an expected cost (the caller's hint, e.g. the Newton iterations of the previous call), so the
 // long integrations start first and do not form a tail.  Bucket = bit length of the hint.
 // ---------------------------------------------------------------------------------------------
-constexpr int NBUCKET = 32;
-__device__ __forceinline__ int cost_bucket(uint32_t c)
-{
-    const int b = c == 0 ? 0 : 32 - __clz(c);
-    return b < NBUCKET ? b : NBUCKET - 1;
-}
 
 // Dispatch key: the cost bucket, plus NBUCKET for a particle routed to the FP64 pass of a mixed
 // batch (nonzero fp64 hint).  Keys are laid out in descending order, so the routed particles form
 // the prefix [0, nH) of the order and the others [nH, n), each longest first.
 constexpr int NKEY = 2 * NBUCKET, BIN_STRIDE = 2 * NKEY + 4; // counts, offsets, range {0, nH, n}
-// A dense particle without a count yet (hint 0: a first step) goes first, as in a call without an
-// order (solve_particles): 60,013 net86 particles, two steps at cap 2,000: 91.2 -> 86.2 ms.
-__device__ __forceinline__ int order_key(const uint32_t* cost, const uint32_t* hint, const double* rho, size_t i)
+__device__ __forceinline__ int order_key(const uint32_t* cost, const uint32_t* hint, const double* rho,
+                                         const double* temp, size_t i)
 {
-    int b = cost ? cost_bucket(cost[i]) : 0;
-    if (b == 0 && rho[i] >= k::denseRho) b = NBUCKET - 1;
-    return (hint && hint[i] != 0u ? NBUCKET : 0) + b;
+    return (hint && hint[i] != 0u ? NBUCKET : 0) +
+           order_bucket(cost ? cost[i] : 0u, rho[i] >= k::denseRho && temp[i] > k::minTemp);
 }
 
 // bins[0 .. NKEY): counts; zeroed by nnet_queue_reset before the launch
 __global__ void __launch_bounds__(256) nnet_order_count(const uint32_t* __restrict__ cost,
-                                                        const uint32_t* __restrict__ hint, const double* __restrict__ rho, size_t n,
-                                                        unsigned* bins)
+                                                        const uint32_t* __restrict__ hint,
+                                                        const double* __restrict__ rho,
+                                                        const double* __restrict__ temp, size_t n, unsigned* bins)
 {
     __shared__ unsigned h[NKEY];
     if (threadIdx.x < NKEY) h[threadIdx.x] = 0u;
     __syncthreads();
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        atomicAdd(&h[order_key(cost, hint, rho, i)], 1u);
+        atomicAdd(&h[order_key(cost, hint, rho, temp, i)], 1u);
     __syncthreads();
     if (threadIdx.x < NKEY && h[threadIdx.x]) atomicAdd(&bins[threadIdx.x], h[threadIdx.x]);
 }
@@ -2162,7 +2155,8 @@ __global__ void nnet_order_offsets(unsigned* bins)
 // each 256-particle tile reserves its key ranges with one atomic per key
 __global__ void __launch_bounds__(256) nnet_order_scatter(const uint32_t* __restrict__ cost,
                                                           const uint32_t* __restrict__ hint,
-                                                          const double* __restrict__ rho, size_t n, unsigned* bins,
+                                                          const double* __restrict__ rho,
+                                                          const double* __restrict__ temp, size_t n, unsigned* bins,
                                                           uint32_t* __restrict__ order)
 {
     __shared__ unsigned h[NKEY], base[NKEY];
@@ -2171,7 +2165,7 @@ __global__ void __launch_bounds__(256) nnet_order_scatter(const uint32_t* __rest
         if (threadIdx.x < NKEY) h[threadIdx.x] = 0u;
         __syncthreads();
         const size_t   i = t0 + threadIdx.x;
-        const int      k = i < n ? order_key(cost, hint, rho, i) : 0;
+        const int      k = i < n ? order_key(cost, hint, rho, temp, i) : 0;
         const unsigned r = i < n ? atomicAdd(&h[k], 1u) : 0u;
         __syncthreads();
         if (threadIdx.x < NKEY && h[threadIdx.x]) base[threadIdx.x] = atomicAdd(&bins[NKEY + threadIdx.x], h[threadIdx.x]);
@@ -2550,10 +2544,11 @@ static const uint32_t* enqueue_order(const nnet_batch& b, int bi, const uint32_t
     order_off += b.n;
     const unsigned blocks = (unsigned)std::min<size_t>((b.n + 255) / 256, 2048);
     hipLaunchKernelGGL(nnet_queue_reset, dim3((BIN_STRIDE + 255) / 256), dim3(256), 0, s, bins, BIN_STRIDE);
-    hipLaunchKernelGGL(nnet_order_count, dim3(blocks), dim3(256), 0, s, b.cost_hint, route, b.rho, b.n, bins);
+    hipLaunchKernelGGL(nnet_order_count, dim3(blocks), dim3(256), 0, s, b.cost_hint, route, b.rho,
+                       (const double*)b.temp, b.n, bins);
     hipLaunchKernelGGL(nnet_order_offsets, dim3(1), dim3(64), 0, s, bins);
-    hipLaunchKernelGGL(nnet_order_scatter, dim3(blocks), dim3(256), 0, s, b.cost_hint, route, b.rho, b.n,
-                       bins, order);
+    hipLaunchKernelGGL(nnet_order_scatter, dim3(blocks), dim3(256), 0, s, b.cost_hint, route, b.rho,
+                       (const double*)b.temp, b.n, bins, order);
     range = bins + 2 * NKEY; // {0, nH, n}
     return order;
 }
