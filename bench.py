@@ -9,10 +9,9 @@ path and the mixed-precision path (FP32 tile LU on MFMA + FP64 iterative refinem
 of iterations that do not refine) each run from the same seeded state; `value` is the mixed path's
 rate and config.mixed_over_fp64 the ratio.
 
-Prints one JSON line: particle-steps/s over the timed steps, the dominant kernel's roofline
-(algorithmic FLOPs from the device Newton-iteration counters: per iteration of an n = d+1
-system, 2n^3/3 + 1.5n^2 - 7n/6 (dense unpivoted LU + solve) + 3d^2 (assembly), divided by the
-kernel time measured with HIP events on the stream the kernel runs on), and the CPU baseline:
+Prints one JSON line: particle-steps/s over the timed steps, the kernel time measured with HIP
+events on the stream the kernel runs on, the Newton iterations the device counts (exact cycles of
+rejected attempts included, which are counted and not run), and the CPU baseline:
 the FP64 CPU restatement of the reference's OpenMP path timed on this host on a bounded sample.
 """
 import argparse
@@ -34,22 +33,16 @@ PEAK_FP64 = 78.6e12  # MI355X dense FP64 (vector and matrix)
 # HBM bytes per particle-step of the solve kernels on the net86 C3 distribution, from rocprofv3
 # --pmc FETCH_SIZE and --pmc WRITE_SIZE runs, scaled by the same counters on a plain 512 MiB device
 # copy (`bench.py --copy-calibration 512`: FETCH_SIZE reads 0.5x and WRITE_SIZE 1.0x of the copied
-# bytes).  FP64 (`--precision fp64 --steps 1 --warmup 0 --no-cpu`, one dispatch): 2 x 4,815,118 KiB
-# fetched + 3,973,413 KiB written.  Mixed (`--precision mixed --steps 1 --warmup 1 --no-cpu`, the
-# hinted step: routed FP64 pass + mixed pass + redo pass): 2 x 6,702,294 KiB fetched + 4,368,279
-# KiB written; per 2,097,152 particles.
-TRAFFIC_BYTES_PER_PARTICLE_STEP = {(3, "fp64"): (2 * 4815117.8 + 3973413.2) * 1024 / 2097152,
-                                   (3, "mixed"): (2 * 6702293.56 + 4368279.28) * 1024 / 2097152}
+# bytes).  FP64 (`--precision fp64 --steps 1 --warmup 0 --no-cpu`, one dispatch): 2 x 6,801,982 KiB
+# fetched + 49,178,802 KiB written, most of both spilled registers.  Mixed (`--precision mixed
+# --steps 1 --warmup 1 --no-cpu`, the hinted step: routed FP64 pass + mixed pass + redo pass):
+# 2 x 7,921,476 KiB fetched + 32,293,289 KiB written; per 2,097,152 particles.
+TRAFFIC_BYTES_PER_PARTICLE_STEP = {(3, "fp64"): (2 * 6801982.0 + 49178801.6) * 1024 / 2097152,
+                                   (3, "mixed"): (2 * 7921475.56 + 32293288.88) * 1024 / 2097152}
 
 # The same for the EOS refresh kernel over the C3 particle set (`--workload helm-eos --steps 2
 # --warmup 0 --no-cpu`): 2 x 755,378 KiB fetched + 81,920 KiB written per 2,097,152 particles.
 EOS_TRAFFIC_BYTES_PER_PARTICLE = {3: (2 * 755378.03 + 81920.0) * 1024 / 2097152}
-
-
-def flops_per_iter(net):
-    d = {14: 14, 86: 86, 87: 87}[net]
-    n = d + 1
-    return 2 * n ** 3 / 3 + 1.5 * n ** 2 - 7 * n / 6 + 3 * d ** 2
 
 
 def device_config(torch, cid, n):
@@ -387,18 +380,16 @@ def main():
         torch.cuda.synchronize()
         wall = time.perf_counter() - t0
         kernel_s = float(np.mean([x.elapsed_time(y) for x, y in ev])) / 1e3
+        # the device's counts are those of running every attempt to its end; whole periods of exact
+        # cycles are counted without being run and retried attempts skip their assembly, so these are
+        # no machine rate
         it_step = newton_total / args.steps
-        flops_per_launch = it_step * flops_per_iter(cfg["net"])
         out = {"particle_steps_per_s": n * args.steps / wall, "ms_per_step": wall / args.steps * 1e3,
-               "kernel_ms": kernel_s * 1e3, "achieved_tflops": flops_per_launch / kernel_s / 1e12,
-               "newton_iters_per_step": it_step, "newton_iters_per_s": it_step / kernel_s,
+               "kernel_ms": kernel_s * 1e3, "counted_newton_iters_per_step": it_step,
                "fp64_resolves_per_step": fp64_total / args.steps,
                "status_per_step": (status_hist / args.steps).tolist(),
                "max_iter_particles_per_step": float(status_hist[4]) / args.steps,
-               "max_iter_share_of_iterations": capped_newton / max(newton_total, 1),
-               # resident workgroups x kernel time / iterations: the mean latency of one Newton
-               # iteration of one particle (the work queue keeps every slot busy until the tail)
-               "iteration_latency_us": slots * kernel_s / max(it_step, 1) * 1e6}
+               "max_iter_share_of_counted": capped_newton / max(newton_total, 1)}
         final = {k: st[k] for k in ("Y", "temp", "status", "newton")}
         return cfg, out, final, snap
 
@@ -441,10 +432,9 @@ def main():
     if "mixed" in res and "fp64" in res:
         conf["mixed_over_fp64"] = res["mixed"]["particle_steps_per_s"] / res["fp64"]["particle_steps_per_s"]
         conf["mixed_vs_fp64_error"] = precision_errors(finals["fp64"], finals["mixed"], cfg)
-    # roofline of the dominant kernel, the FP64 solve (all of the FP64 path's time, and the
-    # routed and redo passes that carry most of the mixed path's)
-    dom = res["fp64"] if "fp64" in res else head
-    achieved = dom["achieved_tflops"] * 1e12
+    # the dominant kernel, the FP64 solve (all of the FP64 path's time, and the routed and redo passes
+    # that carry most of the mixed path's), is bound by the latency of one particle's chain of iterations;
+    # how many it runs is not counted on the device, so the line holds no rate of operations
     tb = TRAFFIC_BYTES_PER_PARTICLE_STEP.get((args.config, "fp64" if "fp64" in res else head_prec))
     out = {
         "metric": "net86 particle-steps/s, mixed vs FP64 on 1 GPU at <=1e-6 rel mass-frac error",
@@ -460,17 +450,10 @@ def main():
         "dtype": "f64" if args.precision == "fp64" else "f32+f64",
         "data": "synthetic",
         "config": conf,
-        "roofline": {"bound": "mfma", "achieved": achieved / 1e12, "peak": PEAK_FP64 / 1e12, "unit": "TFLOP/s",
-                     "frac": achieved / PEAK_FP64, "traffic": tb * n if tb is not None else None,
+        "roofline": {"bound": "latency", "peak": PEAK_FP64 / 1e12, "unit": "TFLOP/s",
+                     "traffic": tb * n if tb is not None else None,
                      "traffic_source": "constant: calibrated rocprofv3 FETCH_SIZE/WRITE_SIZE of the profile run",
-                     "kernel": f"nnet_solve_kernel<{cfg['net']}, HELMHOLTZ, FP64>",
-                     # the kernel is latency x slot bound: iterations/s = slots / iteration latency
-                     # the device's counts are those of running every attempt: whole periods of exact
-                     # cycles are counted, not run
-                     "achieved_from": "counted Newton iterations (exact cycles included)",
-                     "limiter": "latency",
-                     "latency_model": {"resident_slots": slots, "iteration_latency_us": dom["iteration_latency_us"],
-                                       "newton_iters_per_s": dom["newton_iters_per_s"]}},
+                     "kernel": f"nnet_solve_kernel<{cfg['net']}, HELMHOLTZ, FP64>", "resident_slots": slots},
     }
     out["cpu_baseline"] = cpu_baseline(cfg, snap) if snap is not None else None
     print(json.dumps(out), flush=True)
