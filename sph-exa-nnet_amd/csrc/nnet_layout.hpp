@@ -13,9 +13,9 @@ constexpr int MAXSP = 88; // species + 1 of the largest network
 // are 16-byte aligned, and 20 words over 64 LDS banks spread the 16 rows of a tile evenly
 constexpr int PANEL8 = 10;
 
-// The exp / pow values of the six hand-fitted rate groups, evaluated one per lane of a wavefront:
-// level 1, NE1 exps and NP1 pows; level 2, NE2 exps of level-1 results.  They pass through the
-// Jacobian array sJv (N1 + NE2 entries), which is rewritten only after the rate phase.
+// The exp / pow values of the six hand-fitted rate groups, evaluated one per lane of a wavefront and
+// broadcast from there (nnet_dev_rates.hpp): NP1 pows of T, NE1 exps of T, NE2 exps of pow values.
+// (No array holds them: the Jacobian's is kept for the next attempt.)
 namespace spx
 {
 constexpr int NE1 = 36, NP1 = 13, N1 = NE1 + NP1, NE2 = 6;

@@ -180,9 +180,9 @@ __device__ __forceinline__ double pow_count(double x, int n)
 __device__ __forceinline__ double factorial_count(int n) { return n == 2 ? 2. : n == 3 ? 6. : n == 4 ? 24. : 1.; }
 
 // ---------------------------------------------------------------------------------------------
-// Tile LU (the mixed path's FP32 factorization; its triangular solves serve FP64 too).  The
-// augmented (N x N+1) Newton matrix lives in registers as 16x16 tiles in the
-// result layout of v_mfma_f64_16x16x4f64: register v of lane l of a tile holds row 16*I + (l>>4)
+// Tile LU: the mixed path's FP32 factorization and its triangular solves (R = double: the back
+// substitution of the FP64 net86 / net87 solve).  The augmented (N x N+1) Newton matrix lives in
+// registers as 16x16 tiles in the result layout of v_mfma_f64_16x16x4f64: register v of lane l of a tile holds row 16*I + (l>>4)
 // + 4v, column 16*J + (l&15).  Wave (wr, wc) of the WR x WR wave grid owns tiles (wr + WR*ti,
 // wc + WR*tj).  Elimination proceeds in blocks of four pivots (eigen.hpp:182-206 order per
 // element): the owners publish the block's four columns and four rows to LDS; every lane factors
@@ -271,7 +271,7 @@ struct TileT<float>
     }
 };
 
-template<int NET, typename R, bool STORE_L, bool WAVE>
+template<int NET, typename R, bool WAVE>
 struct TileLU
 {
     using C = Cfg<NET>;
@@ -368,13 +368,10 @@ struct TileLU
 #pragma unroll
                 for (int c = q + 1; c < 4; ++c)
                     if (p0 + c <= N) sU[uidx(p0 + q, p0 + c)] = Un[q][c];
-                if constexpr (STORE_L)
-                {
-                    sRinv[p0 + q] = rinv[q];
+                sRinv[p0 + q] = rinv[q];
 #pragma unroll
-                    for (int c = 0; c < q; ++c)
-                        sL[lrow(p0 + q) + p0 + c] = Wt[q][c];
-                }
+                for (int c = 0; c < q; ++c)
+                    sL[lrow(p0 + q) + p0 + c] = Wt[q][c];
             }
         // the last block has no trailing rows; net86 and net14 have no trailing columns there
         // either, so the diagonal block's stores above are all it leaves (wavefront 0 runs the
@@ -405,10 +402,9 @@ struct TileLU
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                     P(i, q) = Lq[q];
-                if constexpr (STORE_L)
 #pragma unroll
-                    for (int q = 0; q < nq; ++q)
-                        sL[lrow(i) + p0 + q] = Lq[q];
+                for (int q = 0; q < nq; ++q)
+                    sL[lrow(i) + p0 + q] = Lq[q];
             }
         }
         else
@@ -448,7 +444,7 @@ struct TileLU
 #pragma unroll
         for (int ti = 0; ti < TI; ++ti)
         {
-            const int i = 16 * (wr + WR * ti) + X::arow(std::is_same<R, float>::value, lc);
+            const int i = 16 * (wr + WR * ti) + X::arow(true, lc);
             Aop[ti]     = (i >= p0 + 4 && i < N) ? -P(i, lr) : R(0);
         }
 #pragma unroll
@@ -484,8 +480,8 @@ struct TileLU
         if constexpr (STEP + 1 < NS) step<STEP + 1>(Mt, pan, sU, sL, sRinv, wr, wc, lr, lc, tid);
     }
 
-    // forward elimination of the augmented matrix; leaves the normalised rows in sU (and, with
-    // STORE_L, the multipliers in sL and the pivot reciprocals in sRinv)
+    // forward elimination of the augmented matrix; leaves the normalised rows in sU, the multipliers
+    // in sL and the pivot reciprocals in sRinv
     static __device__ __forceinline__ void factor(V (&Mt)[TI][TI], R* pan, R* sU, R* sL, R* sRinv, int wr, int wc,
                                                   int lr, int lc, int tid)
     {
@@ -834,10 +830,11 @@ struct PanelLU
         if constexpr (B + 1 < X::NB) step<B + 1>(Mt, pan, sU, w, lane);
     }
 
-    // forward elimination of the augmented matrix; leaves the normalised rows in sU (the caller has
-    // every lane's matrix in its registers: sU overwrites the arrays it was built from)
+    // forward elimination of the augmented matrix; leaves the normalised rows in sU, in front of all that
+    // the fill reads
     static __device__ __forceinline__ void factor(dx4 (&Mt)[TI][TI], double* pan, double* sU, int w, int lane)
     {
+        static_assert(Lds<NET, false>::oBE >= N * (N + 1) / 2, "packed rows below the arrays of the fill");
         __syncthreads();
         publish<0>(Mt, pan, sU, w / WR, w % WR, lane >> 4, lane & 15);
         __syncthreads();
@@ -1002,11 +999,14 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
     const size_t q0 = bd.qrange ? (size_t)bd.qrange[0] : 0, q1 = bd.qrange ? (size_t)bd.qrange[1] : bd.n;
     // Without an order, dense particles first: the queue runs over the particles twice and leaves the
     // others to the second time.  A particle that runs into the iteration cap takes as long as the
-    // rest of the call, and the call as long as both when it is met late.  Such particles are dense:
-    // rho >= 1e7 g/cm^3 holds for all of them on the net86 and net87 Helmholtz sets (30% and all of
-    // the particles) and for 83% on net14's (60%).  Not where every particle starts at once, nor where
-    // much of the batch does not burn (nnet_queue_plan).
-    // 524,288 net86 particles, first step: 364 -> 280 ms; 50,021 of net14 68.5 -> 65.8.
+    // rest of the call, and the call as long as both when it is met late.  Such particles are dense: on
+    // the net86 set all of them have rho >= 1e7 g/cm^3, and 30% of the particles (the set's hot part is
+    // drawn from there up, its cool part from there down, so no other line was tried against it); on
+    // net14's, drawn over all densities, 83% of them and 60% of the particles.  It changes the order
+    // only.  Not where every particle starts at once, nor where much of the batch does not burn
+    // (nnet_queue_plan).  First step, means over eight sets: 524,288 net86 particles 359 -> 333 ms (one
+    // set 383 -> 329, another 365 -> 374: the longest particle alone takes 250 to 390), 50,021 of net14
+    // 69.5 -> 65.1.
     const unsigned nq    = (unsigned)(q1 - q0), // (the host refuses more than queue_limit)
                    times = queue_passes(nq, gridDim.x * groups, bd.order || bd.queue[QPLAN] == 0u);
     for (;;)
@@ -1114,8 +1114,9 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
             }
             if (i == 1) kept = IN_LDS;
             // an opaque lane index (range restored): the lane's addresses are formed in each iteration,
-            // not kept from the kernel's entry and spilled (net86 Helmholtz FP64: 67 -> 19 VGPRs, net14
-            // 137 -> 84; 524,288 net86 particles 568 -> 536 ms, 4,099 of net87 at cap 2,000 95 -> 87 ms)
+            // not kept from the kernel's entry and spilled (when it was made, net86 Helmholtz FP64 67 -> 19
+            // spilled VGPRs, 524,288 particles 568 -> 536 ms, 4,099 of net87 at cap 2,000 95 -> 87 ms; the kept
+            // arrays and the rate passes have brought them to 66 since)
             asm volatile("" : "+v"(tid));
             tid &= NT - 1;
             if (!again)
@@ -1527,16 +1528,10 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
             const double thdt    = k::theta * used_dt;
             const double drho    = drho_dt * used_dt;
             const double value_1 = dpdTv * drho / (rho_t * rho_t);
-            // matrix entry (ri, ci) from the assembly arrays, as prepareSystemFromGuess builds it;
-            // J is the Jacobian entry (0 where the pattern has none)
+            // matrix entry (ri, ci) of a species row, ri >= 1, from the assembly arrays, as
+            // prepareSystemFromGuess builds it; J is the Jacobian entry (0 where the pattern has none)
             auto entry = [&](int ri, int ci, double J) __attribute__((always_inline)) -> double
             {
-                if (ri == 0)
-                {
-                    if (ci == 0) return 1 - k::theta * value_1 / cvv;
-                    if (ci < N) return -sBE[ci - 1] / cvv;
-                    return T * value_1 / cvv;
-                }
                 const int s = ri - 1;
                 if (ci == 0) return sDYT[s] * mthdt;
                 if (ci < N) return (ci == ri) ? 1. - thdt * J : mthdt * J;
@@ -1597,7 +1592,7 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
                             const int ri = tile_row(wr + WR * ti, lr, v);
                             if (ri >= 1 && ri < N) Mt[ti][JN / WR][v] = entry(ri, N, 0.);
                         }
-                // row 0 (temperature): entry()'s three forms with one quotient
+                // row 0 (temperature): 1 - theta v / cv, -BE / cv and T v / cv with one quotient
                 if (wr == 0 && lr == 0)
 #pragma unroll
                     for (int tj = 0; tj < TI; ++tj)
@@ -1636,10 +1631,10 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
                     for (int a = 0; a < NA; ++a)
                     {
                         const int row = tid + 64 * a;
-                        const double x = sU[row < N ? TileLU<NET, double, false, WAVE>::uidx(row, N) : 0];
+                        const double x = sU[row < N ? TileLU<NET, double, WAVE>::uidx(row, N) : 0];
                         acc[a]         = row < N ? x : 0.;
                     }
-                    TileLU<NET, double, false, WAVE>::back(sU, acc, tid);
+                    TileLU<NET, double, WAVE>::back(sU, acc, tid);
                     // (and whether an abundance becomes NaN, for the controller)
                     bool bad = false;
 #pragma unroll
@@ -1667,7 +1662,7 @@ __device__ __forceinline__ void solve_particles(const NetDev& nd, const EosT& ed
                 // ---- mixed precision: FP32 tile LU + FP64 iterative refinement; a particle
                 //      with an iteration whose refinement does not converge is abandoned here
                 //      and integrated again, from the start of the step, by the FP64 pass ----
-                using LU32 = TileLU<NET, float, true, WAVE>;
+                using LU32 = TileLU<NET, float, WAVE>;
                 float* sU32   = reinterpret_cast<float*>(sm);
                 float* sL32   = sU32 + L::NU;
                 float* sRi32  = sL32 + L::NL;
@@ -1966,7 +1961,8 @@ __global__ void __launch_bounds__(FUSE_NT, 2) nnet_solve_fused(FusedDev fd, Step
         // the lane index enters each network's code through an empty asm statement, so the
         // compiler forms each network's lane-dependent values inside its own branch instead of
         // hoisting common ones above the branches, where they would stay live through all three
-        // (fused Helmholtz FP64 kernel: 72 -> 25 spilled VGPRs)
+        // (fused Helmholtz FP64 kernel, when it was made: 72 -> 25 spilled VGPRs; 153 now, against 66 / 65
+        // / 67 of the three networks' own kernels)
         int t = threadIdx.x;
         if (P.kind == 87)
         {
