@@ -9,9 +9,11 @@ reload returns what the scratch memory held.  One build of the fused multi-netwo
 coefficients of its logarithm that way and returned wrong abundances without any error; whether a
 build does depends on its register pressure, so every build is checked.
 
-A block counts as a join if a branch on an empty mask (s_cbranch_execz) leads to it, or if it
-follows a loop's branch on a non-empty one (s_cbranch_execnz): its first instructions may run with
-no lane active, so a vector instruction that only some lanes were to skip cannot be there.
+A block counts as a join if a branch on an empty mask (s_cbranch_execz) leads to it right after
+the mask was narrowed, or if it follows a loop's branch on a non-empty one (s_cbranch_execnz): its
+first instructions may run with no lane active, so a vector instruction that only some lanes were to
+skip cannot be there.  (The compiler also writes branches that are never taken as s_cbranch_execz,
+behind no change of the mask: their targets are ordinary code.)
 
     python3 isa_check.py lib/libnnet_mi355x.so     lists the findings, exit status 1 if any
 """
@@ -29,6 +31,8 @@ _INS = re.compile(r"^\t(\S+)(?: (.*?))?\s*// ([0-9A-F]+):[0-9A-F ]*(?:<([^>+]+)(
 _ANY_LANES = re.compile(r"v_(readlane|writelane|readfirstlane|mfma|nop)")
 # a join gives lanes back: the mask of the branch it ends, or the other side of an if / else
 _RESTORE = re.compile(r"s_or_b64 exec, exec,|s_mov_b64 exec,|s_(or|andn2)_saveexec_b64")
+# the mask loses lanes (an else: what its saveexec form gave back, less the other side)
+_NARROW = re.compile(r"s_(and|andn2|xor)_b64 exec,|s_(and|andn2)_saveexec_b64")
 _VECTOR = re.compile(r"(v|scratch|global|flat|ds|buffer)_")
 
 
@@ -56,13 +60,22 @@ def findings(text):
     number of joins looked at."""
     found, joins = [], 0
     for name, ins in _kernels(text):
-        starts = set()
-        for k, (_, op, _, target) in enumerate(ins):
-            if op == "s_cbranch_execz":
+        starts, narrowed = set(), False
+        targets = {t for _, _, _, t in ins if t is not None}
+        for k, (a, op, args, target) in enumerate(ins):
+            if a in targets:
+                narrowed = False
+            if _NARROW.match(f"{op} {args}"):
+                narrowed = True
+            elif _RESTORE.match(f"{op} {args}"):
+                narrowed = False
+            elif op == "s_cbranch_execz" and narrowed:
                 starts.add(target)
-            elif op == "s_cbranch_execnz" and k + 1 < len(ins):
+            elif op == "s_cbranch_execnz" and narrowed and k + 1 < len(ins):
                 nxt = ins[k + 1]
                 starts.add(nxt[3] if nxt[1] == "s_branch" else nxt[0])
+            if op.startswith(("s_cbranch", "s_branch", "s_setpc")):
+                narrowed = False
         at = {a: k for k, (a, _, _, _) in enumerate(ins)}
         for s in sorted(starts):
             joins += 1

@@ -41,8 +41,8 @@ def test_spills_in_front_of_the_restore(front):
 def test_else_branch_and_lane_moves():
     # the other side of an if / else restores with a saveexec form; register-to-lane moves do not
     # depend on the mask; a narrower branch that starts right away is no restore
-    head = "0000000000001000 <kernel>:\n\ts_cbranch_execz 1     // 000000001000: BF880001 <kernel+0x8>\n"
-    head += "\ts_nop 0               // 000000001004: BF800000\n"
+    head = "0000000000000ffc <kernel>:\n\ts_and_saveexec_b64 s[0:1], vcc   // 000000000FFC: BE80206A\n"
+    head += "\ts_cbranch_execz 1     // 000000001000: BF880001 <kernel+0xc>\n\ts_nop 0       // 000000001004: BF800000\n"
     tail = "\ts_endpgm               // 000000001018: BF810000\n"
     for first, mask, hits in (("v_mov_b32_e32 v1, v2", "s_andn2_saveexec_b64 s[0:1], s[54:55]", 1),
                               ("v_mov_b32_e32 v1, v2", "s_or_saveexec_b64 s[0:1], s[54:55]", 1),
@@ -50,6 +50,23 @@ def test_else_branch_and_lane_moves():
                               ("v_mov_b32_e32 v1, v2", "s_and_saveexec_b64 s[0:1], vcc", 0)):
         text = head + f"\t{first}      // 000000001008: 7E020302\n\t{mask}      // 000000001010: 87FE007E\n" + tail
         assert len(isa_check.findings(text)[0]) == hits, (first, mask)
+
+
+def test_branch_that_is_never_taken():
+    # the compiler writes some branches that are never taken as branches on an empty mask: the mask
+    # was not narrowed for them, and what they lead to is ordinary code in front of a restore
+    text = """
+0000000000001000 <kernel>:
+{0}\ts_nop 0                                                     // 000000001004: BF800000
+\ts_cbranch_execz 1                                           // 000000001008: BF880001 <kernel+0x10>
+\ts_branch 2                                                  // 00000000100C: BF820002 <kernel+0x18>
+\tv_mul_f64 v[18:19], v[4:5], s[0:1]                          // 000000001010: D2810012 00000104
+\ts_or_b64 exec, exec, s[2:3]                                 // 000000001018: 87FE027E
+\ts_endpgm                                                    // 00000000101C: BF810000
+"""
+    for before, hits in (("", 0), ("\ts_and_saveexec_b64 s[2:3], vcc        // 000000001000: BE82206A\n", 1),
+                         ("\ts_or_b64 exec, exec, s[2:3]            // 000000001000: 87FE027E\n", 0)):
+        assert len(isa_check.findings(text.format(before))[0]) == hits, before
 
 
 def test_built_library_has_none():
