@@ -33,12 +33,12 @@ PEAK_FP64 = 78.6e12  # MI355X dense FP64 (vector and matrix)
 # HBM bytes per particle-step of the solve kernels on the net86 C3 distribution, from rocprofv3
 # --pmc FETCH_SIZE and --pmc WRITE_SIZE runs, scaled by the same counters on a plain 512 MiB device
 # copy (`bench.py --copy-calibration 512`: FETCH_SIZE reads 0.5x and WRITE_SIZE 1.0x of the copied
-# bytes).  FP64 (`--precision fp64 --steps 1 --warmup 0 --no-cpu`, one dispatch): 2 x 6,801,982 KiB
-# fetched + 49,178,802 KiB written, most of both spilled registers.  Mixed (`--precision mixed
+# bytes).  FP64 (`--precision fp64 --steps 1 --warmup 0 --no-cpu`, one dispatch): 2 x 6,738,827 KiB
+# fetched + 47,995,497 KiB written, most of it spilled registers.  Mixed (`--precision mixed
 # --steps 1 --warmup 1 --no-cpu`, the hinted step: routed FP64 pass + mixed pass + redo pass):
-# 2 x 7,921,476 KiB fetched + 32,293,289 KiB written; per 2,097,152 particles.
-TRAFFIC_BYTES_PER_PARTICLE_STEP = {(3, "fp64"): (2 * 6801982.0 + 49178801.6) * 1024 / 2097152,
-                                   (3, "mixed"): (2 * 7921475.56 + 32293288.88) * 1024 / 2097152}
+# 2 x 7,870,993 KiB fetched + 31,926,740 KiB written; per 2,097,152 particles.
+TRAFFIC_BYTES_PER_PARTICLE_STEP = {(3, "fp64"): (2 * 6738827.0 + 47995496.6) * 1024 / 2097152,
+                                   (3, "mixed"): (2 * 7870992.63 + 31926740.25) * 1024 / 2097152}
 
 # The same for the EOS refresh kernel over the C3 particle set (`--workload helm-eos --steps 2
 # --warmup 0 --no-cpu`): 2 x 755,378 KiB fetched + 81,920 KiB written per 2,097,152 particles.
