@@ -134,15 +134,18 @@ __attribute__((always_inline)) constexpr uint32_t queue_passes(uint32_t nq, uint
 {
     return !ordered && nq > groups && nq <= (0xffffffffu - groups) / 2 ? 2 : 1;
 }
-// A second pass takes every position again, and positions come at one atomic each (11 ns on one
-// address, however many groups ask), so it is left out where taking positions is most of the call:
-// where many particles do not burn.  `idle` of PLAN_SAMPLE particles spread over the batch do not.
-// Two passes against one: 50,021 net14 particles, all idle, 1.19 ms against 0.63; 1,000,000 of net86,
-// nine in ten idle, 28.6 against 19.8.  With a quarter idle the second pass costs a call of particles
-// that take two iterations each 8% (net86: 11 ns on 145 per position), others less, and a call with
-// capped particles gains more (solve_particles).
+// A second pass takes every position again, and positions come at one atomic each (11.4 ns on one
+// address, however many groups ask), so it is left out where it cannot pay: where half of the particles
+// do not burn and taking positions is much of the call, and where the particles that burn are all of one
+// kind.  Of PLAN_SAMPLE particles spread over the batch `idle` do not burn and `dense` burn and are
+// dense.  Two passes against one: 50,021 net14 particles, all idle, 1.19 ms against 0.63; 1,000,000 of
+// net86, nine in ten idle, 28.6 against 19.8; 100,000 of net86 that take two iterations each, 20 / 50 / 80%
+// of them idle, 14.1 / 9.0 / 4.4 against 13.9 / 8.9 / 3.8.  What it gains with capped particles: solve_particles.
 constexpr uint32_t PLAN_SAMPLE = 256;
-constexpr bool     dense_first_pays(uint32_t idle) { return 4 * idle <= PLAN_SAMPLE; }
+constexpr bool     dense_first_pays(uint32_t idle, uint32_t dense)
+{
+    return 2 * idle <= PLAN_SAMPLE && dense > 0 && idle + dense < PLAN_SAMPLE;
+}
 // Particles of one launch at most, on a device of n_cu compute units (32 wavefronts each).
 constexpr uint64_t queue_limit(uint32_t n_cu) { return 0xffffffffull - 32ull * n_cu; }
 

@@ -2090,15 +2090,15 @@ __global__ void nnet_queue_reset(unsigned int* q, int n)
 
 // The reset of a batch's counters in a call without an order and with more particles than start at
 // once: also decides, from particles spread over the batch, whether dense particles go first
-// (dense_first_pays; one pair of loads per lane, so it takes a plain reset's time and their latency).
+// (dense_first_pays; one pair of loads per lane: a plain reset's time and their latency).
 __global__ void __launch_bounds__(PLAN_SAMPLE)
     nnet_queue_plan(unsigned int* q, int nctr, const double* __restrict__ rho, const double* __restrict__ temp, size_t n)
 {
     const int    i    = threadIdx.x;
     const size_t p    = (size_t)((unsigned long long)n * i / PLAN_SAMPLE);
-    const bool   idle = !(rho[p] > k::minRho && temp[p] > k::minTemp);
-    const int    cnt  = __syncthreads_count(idle);
-    if (i < nctr) q[i] = i == QPLAN && dense_first_pays((unsigned)cnt) ? 1u : 0u;
+    const bool   burns = rho[p] > k::minRho && temp[p] > k::minTemp;
+    const int    idle  = __syncthreads_count(!burns), dense = __syncthreads_count(burns && rho[p] >= k::denseRho);
+    if (i < nctr) q[i] = i == QPLAN && dense_first_pays((unsigned)idle, (unsigned)dense) ? 1u : 0u;
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -27,6 +27,15 @@ int main()
                     if (!ok && n_fail++ < 20)
                         std::printf("FAIL n %lld groups %u ordered %d passes %u\n", (long long)n, groups, ordered, t);
                 }
+    // dense particles first: not where more than half of the sample is idle, nor where all that burns is
+    // dense or none of it is
+    for (uint32_t idle = 0; idle <= PLAN_SAMPLE; ++idle)
+        for (uint32_t dense = 0; idle + dense <= PLAN_SAMPLE; ++dense)
+        {
+            const uint32_t thin = PLAN_SAMPLE - idle - dense;
+            if (dense_first_pays(idle, dense) != (idle <= PLAN_SAMPLE / 2 && dense >= 1 && thin >= 1) && n_fail++ < 20)
+                std::printf("FAIL idle %u dense %u\n", idle, dense);
+        }
     std::printf("%d failures\n", n_fail);
     return n_fail != 0;
 }

@@ -38,7 +38,7 @@ def _call(torch, nm, ctx, cfg, rho, temp, mixed=False, hint=None):
 
 
 @pytest.mark.parametrize("net,mixed", [(14, False), (86, False), (86, True), (87, False)])
-@pytest.mark.parametrize("idle", [0., 0.2, 0.3, 0.9, 1.])
+@pytest.mark.parametrize("idle", [0., 0.2, 0.45, 0.55, 0.9, 1.])
 def test_idle_share_changes_no_result(net, mixed, idle):
     import torch
     if not torch.cuda.is_available():
